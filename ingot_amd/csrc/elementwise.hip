@@ -9,14 +9,6 @@ namespace ingot {
 
 namespace {
 
-__device__ __forceinline__ float load_f(const void* p, int dt, int64_t i) {
-    switch (dt) {
-        case INGOT_DT_F32: return ((const float*)p)[i];
-        case INGOT_DT_BF16: return bf16_to_f32(((const uint16_t*)p)[i]);
-        default: return 0.f;
-    }
-}
-
 __device__ __forceinline__ int32_t load_i(const void* p, int dt, int64_t i) {
     switch (dt) {
         case INGOT_DT_U8: return (int32_t)((const uint8_t*)p)[i];
@@ -33,35 +25,6 @@ inline unsigned grid_for(int64_t work, int per_block) {
     return (unsigned)b;
 }
 
-// dst[j][k] (np × kp, dst_kind) = src element (j, k) of the logical [n][k]
-// weight, zero outside n × k. One thread per destination element.
-__global__ void pack_weight_kernel(const void* src, int src_dt, int64_t ld, int trans, int64_t n, int64_t k,
-                                   void* dst, int dst_kind, int64_t np, int64_t kp, int64_t ldk, int64_t src_item,
-                                   int64_t dst_item) {
-    // blockIdx.y: matrix item (src_item / dst_item elements apart)
-    const int dsz = dst_kind == KIND_I8 ? 1 : (dst_kind == KIND_BF16 ? 2 : 4);
-    const int ssz = src_dt == INGOT_DT_F32 ? 4 : (src_dt == INGOT_DT_BF16 ? 2 : 1);
-    src = (const char*)src + blockIdx.y * src_item * ssz;
-    dst = (char*)dst + blockIdx.y * dst_item * dsz;
-    const int64_t total = np * kp;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t j = t / kp, kk = t - j * kp;
-        const int64_t i = j * ldk + kk;
-        const bool in = j < n && kk < k;
-        const int64_t si = trans ? j * ld + kk : kk * ld + j;
-        if (dst_kind == KIND_I8) {
-            ((int8_t*)dst)[i] = in ? ((const int8_t*)src)[si] : (int8_t)0;
-        } else {
-            const float v = in ? load_f(src, src_dt, si) : 0.f;
-            if (dst_kind == KIND_BF16) {
-                ((uint16_t*)dst)[i] = (in && src_dt == INGOT_DT_BF16) ? ((const uint16_t*)src)[si] : f32_to_bf16(v);
-            } else {
-                ((float*)dst)[i] = v;
-            }
-        }
-    }
-}
-
 // One wave per row: colsum[j] = Σ_k packed[j][k] (int32 wrap-around).
 __global__ void colsum_kernel(const int8_t* packed, int64_t kp, int64_t ldk, int64_t n, int32_t* colsum) {
     const int64_t j = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -73,85 +36,207 @@ __global__ void colsum_kernel(const int8_t* packed, int64_t kp, int64_t ldk, int
     if (lane == 0) colsum[j] = (int32_t)s;
 }
 
-// Packs activations into [m][kl] rows of dst_kind, zero padded beyond k.
-// Each thread produces one 16-byte chunk of a destination row. KIND_BF16X2
-// writes two planes, hi at dst and lo at dst + plane (split_bf16).
-__device__ __forceinline__ float load_a(const char* sb, int src_dt, int trans, int64_t lda, int64_t row, int64_t kk) {
-    const int64_t si = trans ? kk * lda + row : row * lda + kk;
-    return load_f(sb, src_dt, si);
+// ---- operand packs ----
+// One operand matrix (a weight, or a call's activations) becomes rows of the
+// destination kind, k-contiguous, zero past n rows and past k columns. The
+// element types a kind is packed from: S is the source element, D the
+// destination's 16-byte chunk of EPC elements.
+template <int KD> struct PackOf { static constexpr int EPC = KD == KIND_F32 ? 4 : (KD == KIND_I8 ? 16 : 8); };
+
+struct PackArgs {
+    const void* src;
+    int64_t ld;          // source row pitch, elements
+    int64_t n, k;        // logical rows and columns of the destination
+    void* dst;
+    int64_t np, kp, ldk; // written rows and columns (kp a multiple of the chunk), row pitch, elements
+    int64_t plane;       // KIND_BF16X2: elements from the hi plane to the lo plane
+    int64_t src_item, dst_item;  // elements between batch items (blockIdx.y)
+    uint32_t flip;       // KIND_I8: XOR of every source byte inside the matrix (0x80: u8 → s8)
+};
+
+// EPC consecutive elements from p, the first `have` of them inside the matrix
+// (the rest are zero), as f32 (bits kept for a bf16 → bf16 copy) or bytes.
+template <int KD, typename S>
+struct Chunk {
+    static constexpr int EPC = PackOf<KD>::EPC;
+    S v[EPC];
+    __device__ __forceinline__ void load(const S* p, int64_t have) {
+        constexpr int BYTES = EPC * (int)sizeof(S);
+        constexpr int VB = BYTES >= 16 ? 16 : BYTES;
+        if (have >= EPC && (((uintptr_t)p) & (VB - 1)) == 0) {
+            if constexpr (VB == 16) {
+                i32x4_t t[BYTES / 16];
+#pragma unroll
+                for (int i = 0; i < BYTES / 16; ++i) t[i] = ((const i32x4_t*)p)[i];
+                __builtin_memcpy(v, t, BYTES);
+            } else {
+                const uint2 t = *(const uint2*)p;
+                __builtin_memcpy(v, &t, 8);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < EPC; ++e) v[e] = e < have ? p[e] : S(0);
+        }
+    }
+};
+
+__device__ __forceinline__ float pack_f32(float v) { return v; }
+__device__ __forceinline__ float pack_f32(uint16_t v) { return bf16_to_f32(v); }
+__device__ __forceinline__ uint16_t pack_bf16(float v) { return f32_to_bf16(v); }
+__device__ __forceinline__ uint16_t pack_bf16(uint16_t v) { return v; }
+
+// Writes one chunk (kept inside the matrix by `live` elements for the byte flip).
+template <int KD, typename S>
+__device__ __forceinline__ void store_chunk(const S (&v)[PackOf<KD>::EPC], int64_t live, const PackArgs& p, char* d) {
+    constexpr int EPC = PackOf<KD>::EPC;
+    i32x4_t out;
+    if constexpr (KD == KIND_I8) {
+        uint8_t b[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) b[e] = e < live ? (uint8_t)(v[e] ^ p.flip) : (uint8_t)0;
+        __builtin_memcpy(&out, b, 16);
+        *(i32x4_t*)d = out;
+    } else if constexpr (KD == KIND_F32) {
+        float f[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[e] = pack_f32(v[e]);
+        __builtin_memcpy(&out, f, 16);
+        *(i32x4_t*)d = out;
+    } else {
+        uint16_t h[EPC], l[EPC];
+#pragma unroll
+        for (int e = 0; e < EPC; ++e) {
+            if constexpr (KD == KIND_BF16X2)
+                split_bf16(pack_f32(v[e]), h[e], l[e]);
+            else
+                h[e] = pack_bf16(v[e]);
+        }
+        __builtin_memcpy(&out, h, 16);
+        *(i32x4_t*)d = out;
+        if constexpr (KD == KIND_BF16X2) {
+            __builtin_memcpy(&out, l, 16);
+            *(i32x4_t*)(d + p.plane * 2) = out;
+        }
+    }
 }
 
-template <int KD>
-__global__ void pack_a_kernel(const void* src, int src_dt, int64_t lda, int trans, int64_t m, int64_t k,
-                              int64_t src_stride, void* dst, int64_t kl, int64_t dst_stride, int64_t plane) {
-    // grid: x over the 16-byte chunks of a row, y over rows (strided), z over batch items
-    constexpr int EPC = KD == KIND_F32 ? 4 : (KD == KIND_I8 ? 16 : 8);  // elements per chunk
-    const int64_t chunks_per_row = kl / EPC;
-    const int64_t cc = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (cc >= chunks_per_row) return;
-    const int b = blockIdx.z;
-    const char* sb = (const char*)src;
-    const int esz = src_dt == INGOT_DT_F32 ? 4 : (src_dt == INGOT_DT_BF16 ? 2 : 1);
-    sb += (int64_t)b * src_stride * esz;
-    const int esz_d = KD == KIND_F32 ? 4 : (KD == KIND_I8 ? 1 : 2);
-    const int64_t k0 = cc * EPC;
-    for (int64_t row = blockIdx.y; row < m; row += gridDim.y) {
-        char* db = (char*)dst + ((int64_t)b * dst_stride + row * kl + k0) * esz_d;
-        if (KD == KIND_I8) {
-            uint8_t v[16];
+template <int KD> constexpr int pack_esz() { return KD == KIND_F32 ? 4 : (KD == KIND_I8 ? 1 : 2); }
+
+// Source rows are k-contiguous ([n][k]): a thread converts one 16-byte chunk
+// of a destination row, 2^txs threads side by side on a row and 256 >> txs
+// rows per workgroup, so short rows (an attention head) fill a workgroup too
+// and no thread divides.
+template <int KD, typename S>
+__global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p, int txs) {
+    constexpr int EPC = PackOf<KD>::EPC;
+    const int tx = threadIdx.x & ((1 << txs) - 1), ty = threadIdx.x >> txs;
+    const int rows = 256 >> txs;
+    const S* src = (const S*)p.src + (int64_t)blockIdx.y * p.src_item;
+    char* dst = (char*)p.dst + (int64_t)blockIdx.y * p.dst_item * pack_esz<KD>();
+    for (int64_t j = (int64_t)blockIdx.x * rows + ty; j < p.np; j += (int64_t)gridDim.x * rows) {
+        const int64_t kin = j < p.n ? p.k : 0;
+        for (int64_t k0 = (int64_t)tx * EPC; k0 < p.kp; k0 += (int64_t)EPC << txs) {
+            Chunk<KD, S> c;
+            c.load(src + j * p.ld + k0, kin - k0);
+            store_chunk<KD, S>(c.v, kin - k0, p, dst + (j * p.ldk + k0) * pack_esz<KD>());
+        }
+    }
+}
+
+// Source rows are n-contiguous ([k][n]): 64 × 64 tiles transposed through LDS,
+// so that both the reads (along n) and the writes (16-byte chunks along k) are
+// whole lines. One element a thread, read straight into its padded place, the
+// pack took 18.2 µs for 96 items of 128 × 64 f32 (2.4 MB) on MI355X; with this
+// kernel and the items' own rows only, Q·Kᵀ (read in place) and P·V of 96
+// heads of 128 × 64 went from 48.0 to 19.5 µs together.
+template <int KD, typename S>
+__global__ __launch_bounds__(256) void pack_cols_kernel(PackArgs p, int64_t tiles, int tiles_k) {
+    constexpr int EPC = PackOf<KD>::EPC;
+    constexpr int T = 64;
+    // row pitch in elements: an odd number of 4-byte words
+    constexpr int PITCH = T + (sizeof(S) == 4 ? 1 : (sizeof(S) == 2 ? 2 : 4));
+    __shared__ S tile[T * PITCH];
+    const S* src = (const S*)p.src + (int64_t)blockIdx.y * p.src_item;
+    char* dst = (char*)p.dst + (int64_t)blockIdx.y * p.dst_item * pack_esz<KD>();
+    const int tid = threadIdx.x;
+    for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+        const int64_t j0 = t / tiles_k * T, k0 = t % tiles_k * T;
+        // 4 n of one k per thread and step: 16 threads a source row, 16 rows a step
+        const int n4 = (tid & 15) * 4, kr = tid >> 4;
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int64_t kk = k0 + e;
-                uint8_t x = 0;
-                if (kk < k) {
-                    const int64_t si = trans ? kk * lda + row : row * lda + kk;
-                    x = ((const uint8_t*)sb)[si];
-                    if (src_dt == INGOT_DT_U8) x ^= 0x80;
-                }
-                v[e] = x;
-            }
-            i32x4_t out;
-            __builtin_memcpy(&out, v, 16);
-            *(i32x4_t*)db = out;
-        } else if (KD == KIND_F32) {
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = k0 + e < k ? load_a(sb, src_dt, trans, lda, row, k0 + e) : 0.f;
-            i32x4_t out;
-            __builtin_memcpy(&out, v, 16);
-            *(i32x4_t*)db = out;
-        } else {
-            float v[8];
-            if (!trans && src_dt == INGOT_DT_F32 && k0 + 8 <= k && ((row * lda + k0) & 3) == 0 &&
-                (((uintptr_t)sb) & 15) == 0) {
-                const f32x4_t* s4 = (const f32x4_t*)((const float*)sb + row * lda + k0);
-                const f32x4_t lo = s4[0], hi = s4[1];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    v[e] = lo[e];
-                    v[e + 4] = hi[e];
+        for (int i = 0; i < T / 16; ++i) {
+            const int kk = kr + i * 16;
+            const int64_t have = k0 + kk < p.k ? p.n - (j0 + n4) : 0;
+            const S* s = src + (k0 + kk) * p.ld + j0 + n4;
+            S v[4];
+            if (have >= 4 && (((uintptr_t)s) & (4 * sizeof(S) - 1)) == 0) {
+                if constexpr (sizeof(S) == 4) {
+                    const i32x4_t w = *(const i32x4_t*)s;
+                    __builtin_memcpy(v, &w, 16);
+                } else if constexpr (sizeof(S) == 2) {
+                    const uint2 w = *(const uint2*)s;
+                    __builtin_memcpy(v, &w, 8);
+                } else {
+                    const uint32_t w = *(const uint32_t*)s;
+                    __builtin_memcpy(v, &w, 4);
                 }
             } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = k0 + e < k ? load_a(sb, src_dt, trans, lda, row, k0 + e) : 0.f;
+                for (int e = 0; e < 4; ++e) v[e] = e < have ? s[e] : S(0);
             }
-            uint16_t h[8], l[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                if (KD == KIND_BF16X2)
-                    split_bf16(v[e], h[e], l[e]);
-                else
-                    h[e] = f32_to_bf16(v[e]);
-            }
-            i32x4_t out;
-            __builtin_memcpy(&out, h, 16);
-            *(i32x4_t*)db = out;
-            if (KD == KIND_BF16X2) {
-                __builtin_memcpy(&out, l, 16);
-                *(i32x4_t*)(db + plane * esz_d) = out;
-            }
+            for (int e = 0; e < 4; ++e) tile[(n4 + e) * PITCH + kk] = v[e];
         }
+        __syncthreads();
+        constexpr int CPR = T / EPC;  // chunks of a tile row
+        for (int c = tid; c < T * CPR; c += 256) {
+            const int jj = c / CPR, kc = c % CPR * EPC;
+            const int64_t j = j0 + jj, k = k0 + kc;
+            if (j >= p.np || k >= p.kp) continue;
+            S v[EPC];
+#pragma unroll
+            for (int e = 0; e < EPC; ++e) v[e] = tile[jj * PITCH + kc + e];
+            store_chunk<KD, S>(v, j < p.n ? p.k - k : 0, p, dst + (j * p.ldk + k) * pack_esz<KD>());
+        }
+        __syncthreads();
     }
+}
+
+// rows: the source is [n][k], else [k][n].
+template <int KD, typename S>
+hipError_t launch_pack(const PackArgs& p, bool rows, int items, hipStream_t st) {
+    if (p.np <= 0 || p.kp <= 0) return hipSuccess;
+    if (rows) {
+        int txs = 0;
+        while (txs < 8 && ((int64_t)PackOf<KD>::EPC << txs) < p.kp) ++txs;
+        hipLaunchKernelGGL((pack_rows_kernel<KD, S>), dim3(grid_for(p.np, 256 >> txs), items), dim3(256), 0, st, p, txs);
+    } else {
+        const int64_t tiles_k = (p.kp + 63) / 64, tiles = (p.np + 63) / 64 * tiles_k;
+        hipLaunchKernelGGL((pack_cols_kernel<KD, S>), dim3(grid_for(tiles, 1), items), dim3(256), 0, st, p, tiles,
+                           (int)tiles_k);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_pack_kind(GemmKind kind, int src_dtype, const PackArgs& p, bool rows, int items, hipStream_t st) {
+    switch (kind) {
+        case KIND_F32:
+            if (src_dtype == INGOT_DT_F32) return launch_pack<KIND_F32, float>(p, rows, items, st);
+            if (src_dtype == INGOT_DT_BF16) return launch_pack<KIND_F32, uint16_t>(p, rows, items, st);
+            break;
+        case KIND_BF16:
+            if (src_dtype == INGOT_DT_F32) return launch_pack<KIND_BF16, float>(p, rows, items, st);
+            if (src_dtype == INGOT_DT_BF16) return launch_pack<KIND_BF16, uint16_t>(p, rows, items, st);
+            break;
+        case KIND_BF16X2:
+            if (src_dtype == INGOT_DT_F32) return launch_pack<KIND_BF16X2, float>(p, rows, items, st);
+            break;
+        case KIND_I8:
+            if (src_dtype == INGOT_DT_I8 || src_dtype == INGOT_DT_U8) return launch_pack<KIND_I8, uint8_t>(p, rows, items, st);
+            break;
+        default: break;
+    }
+    return hipErrorInvalidValue;
 }
 
 // The common activation pack — f32 rows already dense in whole k-tiles (lda = k = kl, one batch
@@ -234,9 +319,8 @@ __global__ void fill_kernel(uint8_t* d, uint8_t v, size_t bytes) {
 hipError_t launch_pack_weight(const void* src, int src_dtype, int64_t ld, int trans, int64_t n, int64_t k, void* dst,
                               GemmKind dst_kind, int64_t np, int64_t kp, int64_t ldk, hipStream_t st, int items,
                               int64_t src_item, int64_t dst_item) {
-    hipLaunchKernelGGL(pack_weight_kernel, dim3(grid_for(np * kp, 256), items), dim3(256), 0, st, src, src_dtype, ld,
-                       trans, n, k, dst, (int)dst_kind, np, kp, ldk, src_item, dst_item);
-    return hipGetLastError();
+    const PackArgs p = {src, ld, n, k, dst, np, kp, ldk, 0, src_item, dst_item, 0u};
+    return launch_pack_kind(dst_kind, src_dtype, p, trans != 0, items, st);
 }
 
 hipError_t launch_colsum_i8(const int8_t* packed, int64_t kp, int64_t ldk, int64_t n, int32_t* colsum,
@@ -248,7 +332,6 @@ hipError_t launch_colsum_i8(const int8_t* packed, int64_t kp, int64_t ldk, int64
 hipError_t launch_pack_a(const void* src, int src_dtype, int64_t lda, int trans, int64_t m, int64_t k,
                          int64_t src_stride, void* dst, GemmKind dst_kind, int64_t kl, int64_t dst_stride, int batch,
                          hipStream_t st) {
-    const int epc = dst_kind == KIND_F32 ? 4 : (dst_kind == KIND_I8 ? 16 : 8);
     // (large activations only: at decode sizes the per-row grid below spreads the few rows over more CUs;
     // M = 16, K = 2048 took 5.4 us flat against 3.7)
     if ((dst_kind == KIND_BF16 || dst_kind == KIND_BF16X2) && src_dtype == INGOT_DT_F32 && !trans && batch == 1 &&
@@ -265,28 +348,9 @@ hipError_t launch_pack_a(const void* src, int src_dtype, int64_t lda, int trans,
                                (uint16_t*)dst, groups, m * kl);
         return hipGetLastError();
     }
-    const int64_t chunks = kl / epc;
-    dim3 grid((unsigned)((chunks + 255) / 256), (unsigned)(m < 65535 ? (m > 0 ? m : 1) : 65535), batch);
-    const int64_t plane = m * kl;
-    switch (dst_kind) {
-        case KIND_BF16:
-            hipLaunchKernelGGL(pack_a_kernel<KIND_BF16>, grid, dim3(256), 0, st, src, src_dtype, lda, trans, m, k,
-                               src_stride, dst, kl, dst_stride, plane);
-            break;
-        case KIND_BF16X2:
-            hipLaunchKernelGGL(pack_a_kernel<KIND_BF16X2>, grid, dim3(256), 0, st, src, src_dtype, lda, trans, m, k,
-                               src_stride, dst, kl, dst_stride, plane);
-            break;
-        case KIND_F32:
-            hipLaunchKernelGGL(pack_a_kernel<KIND_F32>, grid, dim3(256), 0, st, src, src_dtype, lda, trans, m, k,
-                               src_stride, dst, kl, dst_stride, plane);
-            break;
-        case KIND_I8:
-            hipLaunchKernelGGL(pack_a_kernel<KIND_I8>, grid, dim3(256), 0, st, src, src_dtype, lda, trans, m, k,
-                               src_stride, dst, kl, dst_stride, plane);
-            break;
-    }
-    return hipGetLastError();
+    const PackArgs p = {src, lda, m, k, dst, m, kl, kl, m * kl, src_stride, dst_stride,
+                        src_dtype == INGOT_DT_U8 ? 0x80u : 0u};
+    return launch_pack_kind(dst_kind, src_dtype, p, trans == 0, batch, st);
 }
 
 hipError_t launch_dequant(const void* x, int x_dtype, int64_t n, const float* scale, int64_t n_scale, int64_t inner,

@@ -607,6 +607,15 @@ int ingot_rocm_gemv_bf16(ingot_rocm_session* s, const ingot_rocm_gemm_args* a) {
     return run_gemv(s, a, a->w);
 }
 
+// Decode rows take the GEMV: all of M <= 4, and M = 5..16 for N < 4096. At
+// M = 5..16 the wider products run faster as a GEMM of four-stage 32×32
+// tiles (on MI355X at K = 2048, M = 8 and 16: N = 6144 10.7 vs 12.7 µs, N =
+// 11264 13.1 vs 16.2 µs; N = 2048 the GEMV stays ahead, 8.7 vs 10.4 µs).
+static bool gemv_route(const ingot_rocm_session* s, const ingot_rocm_gemm_args* a, GemmKind kind) {
+    return kind == KIND_BF16 && a->M <= 16 && (a->M <= 4 || a->N < 4096) && !a->trans_a &&
+           a->a_dtype == INGOT_DT_F32 && a->batch <= 1 && !s->no_gemv;
+}
+
 // The GEMM after validation. w may be a session weight or a per-call packed
 // operand; stride_b_bytes advances it per batch item (0: shared).
 static int run_gemv_i8g(ingot_rocm_session* s, const ingot_rocm_gemm_args* a, const ingot_rocm_weight* w,
@@ -618,13 +627,7 @@ static int gemm_core(ingot_rocm_session* s, const ingot_rocm_gemm_args* a, const
     const int64_t batch = std::max<int64_t>(1, a->batch);
     if (a->M == 0 || a->N == 0) return INGOT_OK;
     if (w->kind == KIND_I8G) return run_gemv_i8g(s, a, w, noalloc);
-    // Decode rows take the GEMV: all of M <= 4, and M = 5..16 for N < 4096. At
-    // M = 5..16 the wider products run faster as a GEMM of four-stage 32×32
-    // tiles (on MI355X at K = 2048, M = 8 and 16: N = 6144 10.7 vs 12.7 µs, N =
-    // 11264 13.1 vs 16.2 µs; N = 2048 the GEMV stays ahead, 8.7 vs 10.4 µs).
-    if (w->kind == KIND_BF16 && a->M <= 16 && (a->M <= 4 || a->N < 4096) && !a->trans_a &&
-        a->a_dtype == INGOT_DT_F32 && batch == 1 && !s->no_gemv)
-        return run_gemv(s, a, w, noalloc);
+    if (gemv_route(s, a, w->kind)) return run_gemv(s, a, w, noalloc);
 
     // bf16 weights with f32 activations: two bf16 planes (f32-class accuracy)
     // unless the caller asked for single bf16 rounding (INGOT_MATH_BF16).
@@ -643,13 +646,13 @@ static int gemm_core(ingot_rocm_session* s, const ingot_rocm_gemm_args* a, const
     // Every GEMM operand is addressed with 32-bit buffer offsets.
     // Row offsets of a whole tile past the last row (256 rows) must stay below
     // 2^31 too: the kernel marks past-the-end k-tiles by adding 2^31.
-    const int64_t b_extent = w->np * w->ldk * esz;
+    const int64_t b_size = w->np * w->ldk * esz;
     const int64_t a_pitch = direct ? a->lda * a_esz : kl * esz;
     const int64_t a_extent = direct ? (a->M - 1) * a_pitch + kl * esz : (int64_t)planes * a->M * kl * esz;
-    if (b_extent + 256 * w->ldk * esz >= ((int64_t)1 << 31) || a_extent + 256 * a_pitch >= ((int64_t)1 << 31))
+    if (b_size + 256 * w->ldk * esz >= ((int64_t)1 << 31) || a_extent + 256 * a_pitch >= ((int64_t)1 << 31))
         return fail(INGOT_EDECLINED, "gemm: operand larger than 2 GiB");
     g.a_bytes = (uint32_t)a_extent;
-    g.b_bytes = (uint32_t)b_extent;
+    g.b_bytes = (uint32_t)(((w->np - 1) * w->ldk + kl) * esz);  // to the last row's last k-tile
     if (direct) {
         g.a = (const char*)a->d_a;
         g.lda_bytes = a->lda * a_esz;
@@ -685,7 +688,7 @@ static int gemm_core(ingot_rocm_session* s, const ingot_rocm_gemm_args* a, const
     // stay cached between uses: the product's own output and its neighbours'
     // evict them, so they come from HBM, where the tile whose loads are issued
     // two k-tiles ahead is faster (the configuration tables give the figures).
-    if (s->force_gemm_cfg < 0 && c[cfg].deep >= 0 && batch * a_extent + b_extent > kCacheResidentBytes)
+    if (s->force_gemm_cfg < 0 && c[cfg].deep >= 0 && batch * a_extent + b_size > kCacheResidentBytes)
         cfg = c[cfg].deep;
     g.tiles_m = (int)((a->M + c[cfg].bm - 1) / c[cfg].bm);
     g.tiles_n = (int)((a->N + c[cfg].bn - 1) / c[cfg].bn);
@@ -756,15 +759,42 @@ int ingot_rocm_gemm_dynamic_b(ingot_rocm_session* s, const ingot_rocm_gemm_args*
     wt.pack_dtype = f32 ? INGOT_DT_F32 : INGOT_DT_BF16;
     wt.n = a->N;
     wt.k = a->K;
-    wt.np = round_up(a->N, 256);
-    wt.kp = round_up(a->K, 256);
-    wt.ldk = wt.kp + 128 / kind_size(wt.kind);
+    const int esz = kind_size(wt.kind), kt = ktile_elems(wt.kind);
     const int64_t batch = std::max<int64_t>(1, a->batch);
-    const int items = stride_b ? (int)batch : 1;
-    const int64_t item = wt.np * wt.ldk;
     rc = validate_gemm(s, a, &wt);
     if (rc) return rc;
-    wt.data = pool_get(s, (size_t)(items * item * kind_size(wt.kind)));
+    // The limit is that of a B packed like a constant weight, whichever form it takes below.
+    const int64_t lim = (int64_t)1 << 31;
+    const int64_t np = round_up(a->N, 256), kp = round_up(a->K, 256), ldk = kp + 128 / esz;
+    const bool gemv = gemv_route(s, a, wt.kind);
+    if (!gemv && (np + 256) * ldk * esz >= lim) return fail(INGOT_EDECLINED, "gemm: operand larger than 2 GiB");
+    // B rows that are already k-contiguous, of the math type, in whole k-tiles
+    // and 16-byte aligned are what the GEMM's operand loads read (rows past N
+    // lie past the operand's end and load as zero): no pack at all, unless Y
+    // is written over B.
+    const char *b0 = (const char*)d_b, *y0 = (const char*)a->d_y;
+    const char* b1 = b0 + ((batch - 1) * stride_b + (a->N - 1) * ldb + a->K) * esz;
+    const char* y1 = y0 + ((batch - 1) * a->stride_y + (a->M - 1) * a->ldy + a->N) * 4;
+    const bool direct = !gemv && trans_b && (b_dtype == INGOT_DT_F32) == f32 && a->K % kt == 0 && (ldb * esz) % 16 == 0 &&
+                        aligned16(d_b) && (stride_b * esz) % 16 == 0 && (a->N + 256) * ldb * esz < lim &&
+                        (b1 <= y0 || y1 <= b0);
+    if (direct) {
+        wt.data = const_cast<void*>(d_b);
+        wt.np = a->N;
+        wt.kp = a->K;
+        wt.ldk = ldb;
+        return gemm_core(s, a, &wt, stride_b * esz);
+    }
+    // Otherwise each item is packed: for the GEMM only its N rows, in whole
+    // k-tiles (a constant weight's padding to 256 × 256 made the pack of 96
+    // attention heads of 128 × 64 write eight times their bytes), for the GEMV
+    // the padded form it streams.
+    wt.np = gemv ? np : a->N;
+    wt.kp = gemv ? kp : round_up(a->K, kt);
+    wt.ldk = wt.kp + 128 / esz;
+    const int items = stride_b ? (int)batch : 1;
+    const int64_t item = wt.np * wt.ldk;
+    wt.data = pool_get(s, (size_t)(items * item * esz));
     if (!wt.data) return fail(INGOT_ENOMEM, "gemm_dynamic_b: cannot allocate the packed B");
     hipError_t e = launch_pack_weight(d_b, b_dtype, ldb, trans_b ? 1 : 0, a->N, a->K, wt.data, wt.kind, wt.np, wt.kp,
                                       wt.ldk, s->stream, items, stride_b, item);
@@ -772,7 +802,7 @@ int ingot_rocm_gemm_dynamic_b(ingot_rocm_session* s, const ingot_rocm_gemm_args*
         pool_put(s, wt.data);
         return hip_fail(e, "pack B");
     }
-    rc = gemm_core(s, a, &wt, stride_b ? item * kind_size(wt.kind) : 0);
+    rc = gemm_core(s, a, &wt, stride_b ? item * esz : 0);
     pool_put(s, wt.data);  // stream-ordered: later users of the buffer queue behind this GEMM
     return rc;
 }

@@ -244,6 +244,69 @@ def test_gemm_dynamic_b(sess, trans_b, b_dt, shared):
         assert_close(got[i], want, nstar_tol(k, a, bi), f"dynamic b item {i}")
 
 
+@pytest.mark.parametrize("b_dt", ["f32", "bf16"])
+@pytest.mark.parametrize("m,n,k,pad", [(70, 50, 64, 0), (17, 257, 128, 8), (130, 1, 64, 16), (33, 64, 192, 8), (128, 128, 64, 0)])
+def test_gemm_dynamic_b_in_place(sess, b_dt, m, n, k, pad):
+    """[N,K] items read in place (whole k-tiles, 16-byte rows) give the bits of the packed form of the same values
+    ([K,N] items, and [N,K] rows whose pitch is off 16 bytes), with N off the tile grid and NaN past every row."""
+    announce(f"gemm dynamic b in place {b_dt} {m}x{n}x{k} pad={pad}")
+    rng = np.random.default_rng(m * 7 + n + k)
+    bsz = 3
+    a = rng.uniform(-1, 1, (bsz, m, k)).astype(np.float32)
+    bt = rng.uniform(-1, 1, (bsz, n, k)).astype(np.float32)
+    bits = oracle.f32_to_bf16(bt) if b_dt == "bf16" else bt
+    if b_dt == "bf16":
+        bt = oracle.bf16_to_f32(bits)
+    nan = np.array(0x7FC0, np.uint16) if b_dt == "bf16" else np.float32(np.nan)
+    code = L.DT_BF16 if b_dt == "bf16" else None
+
+    def product(rows, cols, vals, trans, ldb_pad):
+        b = np.full((bsz, rows, cols + ldb_pad), nan, vals.dtype)
+        b[:, :, :cols] = vals
+        y = sess.empty(L.DT_F32, (bsz, m, n))
+        sess.gemm_dynamic_b(sess.to_device(a), sess.to_device(b, code), y, m, n, k, trans, cols + ldb_pad,
+                            rows * (cols + ldb_pad), batch=bsz, stride_a=m * k, stride_y=m * n)
+        return y.numpy()
+
+    got = product(n, k, bits, True, pad)
+    np.testing.assert_array_equal(got, product(n, k, bits, True, pad + 3))
+    np.testing.assert_array_equal(got, product(k, n, np.ascontiguousarray(bits.transpose(0, 2, 1)), False, 0))
+    for i in range(bsz):
+        assert_close(got[i], oracle.gemm(a[i], bt[i], trans_b=True), nstar_tol(k, a, bt), f"in place item {i}")
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (63, 65), (64, 64), (65, 63), (130, 257), (257, 128)])
+def test_weight_pack_orders(sess, n, k):
+    """A weight packed from [K,N] (transposed through LDS tiles) and from [N,K] gives the same product bits, for
+    every packed type, at the edges of the 64-wide tiles; so does an A stored [K,M]."""
+    announce(f"weight pack orders {n}x{k}")
+    rng = np.random.default_rng(n * 31 + k)
+    m = 66
+    a = rng.uniform(-1, 1, (m, k)).astype(np.float32)
+    w = rng.uniform(-1, 1, (n, k)).astype(np.float32)
+    da, dat = sess.to_device(a), sess.to_device(np.ascontiguousarray(a.T))
+    for src, pack, code in [(w, L.DT_F32, None), (w, L.DT_BF16, None), (oracle.f32_to_bf16(w), L.DT_BF16, L.DT_BF16)]:
+        ys = []
+        for vals, trans in ((src, True), (np.ascontiguousarray(src.T), False)):
+            wt = sess.upload_weight(vals, trans=trans, pack_dtype=pack, src_dtype=code)
+            for x, ta in ((da, False), (dat, True)):
+                y = sess.empty(L.DT_F32, (m, n))
+                sess.gemm(x, wt, y, m, trans_a=ta)
+                ys.append(y.numpy())
+            wt.free()
+        wf = w if pack == L.DT_F32 else oracle.bf16_to_f32(oracle.f32_to_bf16(w))
+        assert_close(ys[0], oracle.gemm(a, wf, trans_b=True), nstar_tol(k, a, wf), f"pack {pack}")
+        for y in ys[1:]:
+            np.testing.assert_array_equal(y, ys[0])
+    qa = rng.integers(0, 256, (m, k)).astype(np.uint8)
+    qw = rng.integers(-127, 128, (k, n)).astype(np.int8)
+    for vals, trans in ((qw, False), (np.ascontiguousarray(qw.T), True)):
+        wt = sess.upload_weight(vals, trans=trans, pack_dtype=L.DT_I8)
+        y = sess.empty(L.DT_I32, (m, n))
+        sess.matmul_integer(sess.to_device(qa, L.DT_U8), wt, m, 131, y_i32=y)
+        np.testing.assert_array_equal(y.numpy(), oracle.matmul_integer(qa, qw, 131))
+
+
 def test_gemm_dynamic_b_decode_route(sess):
     """M <= 16, one item, bf16 B: the per-call packed B takes the GEMV route."""
     announce("gemm dynamic b gemv route")
