@@ -945,6 +945,13 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
     const int64_t kgl = round_up(K, 128);
     const bool gemm = path == 2 || (path != 1 && Mg >= 16 && K >= 32);
     if (!gemm) {
+        if (path != 1) {
+            bool done = false;
+            hipError_t e = launch_qconv_depthwise(a->d_x, u8 ? 1 : 0, g, (const int8_t*)w->data, w->ldk, a->d_bias,
+                                                  a->d_mult, a->zx, (float)a->zy, yu8, a->d_y, s->stream, &done);
+            if (e != hipSuccess) return hip_fail(e, "qconv depthwise");
+            if (done) return INGOT_OK;
+        }
         hipError_t e = launch_qconv_direct(a->d_x, u8 ? 1 : 0, g, (const int8_t*)w->data, w->ldk, a->d_bias,
                                            a->d_mult, a->zx, (float)a->zy, yu8, a->d_y, s->stream);
         if (e != hipSuccess) return hip_fail(e, "qconv direct");

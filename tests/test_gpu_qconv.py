@@ -134,6 +134,44 @@ def test_routes_agree_at_size(env_session):
     assert len(np.unique(y_gemm)) > 64
 
 
+# Depthwise strips: output widths around groups of 4, one-pixel planes, strips that split a plane and rows long
+# enough to shrink them, kernel rows of one and two words, strides 1, 2 and 3, dilated kernel rows, pads wider than a
+# word, a channel multiplier, 4 x 4 blocks that run over planes; then forms the strip kernel hands to the direct one (9 taps a row, dilated columns).
+DEPTHWISE_CASES = [
+    # n, groups, h, w, multiplier, kh, kw, strides, dilations, pads
+    (2, 5, 57, 55, 1, 3, 3, (1, 1), (1, 1), (1, 1, 1, 1)),
+    (3, 40, 8, 8, 1, 3, 3, (1, 1), (1, 1), (1, 1, 1, 1)),
+    (2, 9, 13, 9, 2, 5, 5, (2, 2), (1, 1), (2, 2, 2, 2)),
+    (1, 6, 10, 17, 1, 5, 5, (1, 1), (1, 1), (9, 11, 4, 12)),
+    (1, 6, 21, 22, 1, 3, 3, (2, 2), (1, 1), (1, 9, 1, 10)),
+    (1, 300, 8, 9, 1, 3, 3, (2, 2), (1, 1), (0, 0, 0, 0)),
+    (1, 3, 56, 56, 1, 3, 3, (2, 2), (1, 1), (0, 0, 1, 1)),
+    (1, 7, 7, 7, 1, 5, 5, (1, 1), (1, 1), (2, 2, 2, 2)),
+    (1, 4, 9, 3, 2, 3, 3, (1, 1), (1, 1), (1, 1, 1, 1)),
+    (1, 2, 1, 1, 3, 1, 1, (1, 1), (1, 1), (0, 0, 0, 0)),
+    (1, 2, 31, 30, 1, 5, 7, (2, 2), (1, 1), (2, 3, 2, 3)),
+    (1, 3, 20, 21, 1, 3, 3, (1, 3), (3, 1), (3, 1, 3, 1)),
+    (1, 2, 8, 6, 1, 2, 8, (1, 1), (1, 1), (0, 6, 1, 7)),
+    (1, 1, 40, 3001, 1, 3, 3, (1, 1), (1, 1), (1, 1, 1, 1)),
+    (1, 1, 5, 9000, 1, 3, 3, (1, 2), (1, 1), (1, 1, 1, 1)),
+    (1, 2, 12, 14, 1, 2, 9, (1, 1), (1, 1), (0, 4, 1, 4)),
+    (1, 2, 12, 14, 1, 3, 3, (1, 1), (2, 2), (2, 2, 2, 2)),
+]
+
+
+@pytest.mark.parametrize("case", DEPTHWISE_CASES, ids=[f"d{i}" for i in range(len(DEPTHWISE_CASES))])
+def test_depthwise_strips(sess, case):
+    n, g, h, w, mult_c, kh, kw, st, dl, pads = case
+    announce(f"qconv depthwise {case}")
+    rng = np.random.default_rng(sum(case[:7]))
+    for x_dtype, zx, y_u8, zy, with_bias in [(np.uint8, 131, True, 9, True), (np.uint8, 0, False, 0, False),
+                                             (np.int8, -128, False, -5, True), (np.int8, 127, True, 128, False)]:
+        x, zx, wt, bias, mult, *_ = make_case(rng, n, g, h, w, g * mult_c, kh, kw, g, x_dtype, zx, with_bias)
+        kw_ = dict(group=g, strides=st, dilations=dl, pads=pads)
+        got = run_conv(sess, x, zx, wt, bias, mult, zy, y_u8, **kw_)
+        np.testing.assert_array_equal(got, oracle.qlinear_conv(x, zx, wt, bias, mult, zy, y_u8, **kw_))
+
+
 def test_empty_and_degenerate(sess):
     announce("qconv empty")
     rng = np.random.default_rng(0)
