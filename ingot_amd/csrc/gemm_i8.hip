@@ -12,6 +12,7 @@ hipError_t launch_gemm_i8(int cfg, const GemmArgs& a, int batch, hipStream_t st)
         case 3: return launch_one<KIND_I8, 64, 64, 2, 2, 2>(a, batch, st);
         case 4: return launch_one<KIND_I8, 64, 96, 2, 2, 2>(a, batch, st);
         case 5: return launch_one<KIND_I8, 32, 32, 2, 2, 4>(a, batch, st);
+        case 6: return launch_one<KIND_I8, 64, 64, 2, 2, 4>(a, batch, st);
     }
     return hipErrorInvalidValue;
 }

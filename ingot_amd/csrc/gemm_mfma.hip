@@ -53,8 +53,12 @@ const GemmConfig kF32Cfgs[] = {{128, 128, 2, 0.90f}, {128, 64, 3, 0.95f}, {64, 6
 // 64×192, 32-row tiles (32×32 to 32×128) and deeper rings were slower there.
 // int8 32×32 with a four-stage ring, for products whose tiles are all resident
 // at once: M = 1–128 at K = 768–2048 took 3.8–5.3 µs instead of 4.7–6.9.
+// int8 64×64 with a four-stage ring, likewise (the pixel GEMM of 256 × 56 × 56 →
+// 256, 3 × 3: 196 tiles of 18 k-tiles, 9.8–10.4 µs instead of 13.2–14.1 with two
+// stages and 11.0 with 32×32; eight stages 10.1–11.4, eight waves 10.7: with the
+// ring this deep a k-tile costs its own operand traffic, not its latency).
 const GemmConfig kI8Cfgs[] = {{256, 256, 1, 1.00f}, {128, 128, 2, 0.60f}, {128, 64, 3, 0.70f}, {64, 64, 4, 1.00f},
-                              {64, 96, 3, 1.06f}, {32, 32, 4, 0.60f, true}};
+                              {64, 96, 3, 1.06f}, {32, 32, 4, 0.60f, true}, {64, 64, 2, 1.20f, true}};
 
 }  // namespace
 
@@ -75,7 +79,7 @@ hipError_t launch_gemm(GemmKind kind, int cfg, const GemmArgs& a, int batch, hip
         case KIND_BF16: return launch_gemm_bf16(cfg, a, batch, st);
         case KIND_BF16X2: return launch_gemm_bf16x2(cfg, a, batch, st);
         case KIND_F32: return launch_gemm_f32(cfg, a, batch, st);
-        case KIND_I8: return launch_gemm_i8(cfg, a, batch, st);
+        case KIND_I8: return a.conv.cpc ? launch_gemm_i8_conv(cfg, a, batch, st) : launch_gemm_i8(cfg, a, batch, st);
         default: break;
     }
     return hipErrorInvalidValue;

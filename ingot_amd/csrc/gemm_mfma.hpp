@@ -171,8 +171,9 @@ __device__ __forceinline__ void waitcnt_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC
 // land on 16 distinct 16-byte bank groups of a 256-byte bank line.
 __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
 
-template <int KD> struct KernelArgs { typedef GemmArgsF type; };
-template <> struct KernelArgs<KIND_I8> { typedef GemmArgsQ type; };
+template <int KD, bool CONV> struct KernelArgs { typedef GemmArgsF type; };
+template <> struct KernelArgs<KIND_I8, false> { typedef GemmArgsQ type; };
+template <> struct KernelArgs<KIND_I8, true> { typedef GemmArgsConv type; };
 
 // RS = 0: k-tiles move global → LDS by DMA into the NS-stage ring (with two
 // stages each load is issued one k-tile ahead of its use). RS = 2 (two-stage
@@ -183,8 +184,15 @@ template <> struct KernelArgs<KIND_I8> { typedef GemmArgsQ type; };
 // coming from HBM need, e.g. behind a cache full of another kernel's output
 // (on MI355X a three-stage ring took the DiT MLP-down tile shape from +32%
 // to +12% over its warm-cache time).
-template <int KD, int BM, int BN, int WGM, int WGN, int NS, int RS = 0>
-__global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename KernelArgs<KD>::type p) {
+//
+// CONV (int8): the rows of A are the output pixels of a convolution and are
+// never written down. The activations lie channel-innermost with their padding
+// (see ConvRows), so the 16-byte chunk q of a row is 16 channels of one tap, at
+// (the pixel's first tap) + (an offset that depends on q alone): each lane adds
+// the offset of its chunk, from a table the workgroup builds in LDS, to the
+// offsets of its rows, which it computes once.
+template <int KD, int BM, int BN, int WGM, int WGN, int NS, int RS = 0, bool CONV = false>
+__global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename KernelArgs<KD, CONV>::type p) {
     // The hi/lo kind (A = hi + lo, two bf16 planes) sums each k-tile in one
     // order on every tile: hi first half, hi second half, lo first half, lo
     // second half. Tiles over 128 rows run it as a bf16 GEMM over twice the
@@ -217,7 +225,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
     constexpr int ECOLS = KD == KIND_I8 ? 3 : 1;
     constexpr int EROWS = KD == KIND_I8 ? 1 : BM;
     static_assert(64 * WGM * WGN >= BN && 64 * WGM * WGN >= EROWS, "one thread per staged column and row");
-    constexpr int EXTRA = (ECOLS * BN + EROWS) * 4;
+    constexpr int TABLE = CONV ? CONV_CHUNKS * 4 : 0;
+    constexpr int EXTRA = (ECOLS * BN + EROWS) * 4 + TABLE;
     // Stages larger than 32 KiB start on 64 KiB boundaries when the ring still
     // fits (a stage straddling a 64 KiB boundary slowed the k-loop on MI355X).
     constexpr int SSTRIDE = STAGE > 32768 && NS * 65536 + EXTRA <= 160 * 1024 ? 65536 : STAGE;
@@ -232,6 +241,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
     __shared__ __attribute__((aligned(1024))) char lds[RING + EXTRA];
     uint32_t(*ep_col)[BN] = (uint32_t(*)[BN])(lds + RING);
     float* ep_row = (float*)(lds + RING + ECOLS * BN * 4);
+    uint32_t* chunk_ofs = (uint32_t*)(lds + RING + EXTRA - TABLE);
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -268,6 +278,30 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
         voff_b[h] = (uint32_t)(lr * p.ldb_bytes) + (uint32_t)(c << 4);
     }
 
+    // CONV: the byte offset of this lane's row of each DMA instruction, and of
+    // its chunk of the next k-tile to load (NW is even, so a lane has one chunk
+    // position for all its rows). Rows past M start past the buffer's end, as
+    // do chunks past the last tap (their weights are zero).
+    static_assert(!CONV || (KD == KIND_I8 && RS == 0 && NW % 2 == 0), "CONV: int8, DMA ring");
+    uint32_t pix[CONV ? IA : 1], tofs = 0;
+    const uint32_t* lane_ofs = chunk_ofs + (lp ^ swz((wave & 1) * 8 + lr));
+    if constexpr (CONV) {
+        const ConvRows& c = p.conv;
+        for (int q = tid; q < (p.kt + NS + 1) * 8; q += 64 * NW) {
+            const int tap = q / c.cpc, kh = tap / c.kw;
+            chunk_ofs[q] = tap < c.taps ? (uint32_t)(kh * c.kh_bytes + (tap - kh * c.kw) * c.kw_bytes + (q - tap * c.cpc) * 16)
+                                        : 0x80000000u;
+        }
+#pragma unroll
+        for (int j = 0; j < IA; ++j) {
+            const int m = m0 + (j * NW + wave) * 8 + lr;
+            const int img = m / c.p, px = m - img * c.p, oh = px / c.ow;
+            pix[j] = m < p.M ? (uint32_t)(img * c.img_bytes + oh * c.oh_bytes + (px - oh * c.ow) * c.ow_bytes) : 0x80000000u;
+        }
+        __syncthreads();
+        tofs = lane_ofs[0];
+    }
+
     // The whole byte offset (row, plane, k-tile, lane chunk) goes in the
     // range-checked VGPR offset; the SGPR offset stays 0. A k-tile index past
     // the end gets offset 2^31 + row offset (< 2^32, above every extent: the
@@ -286,10 +320,15 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
 #pragma unroll
             for (int j = 0; j < IA; ++j) {
                 const int r = (j * NW + wave) * 8;
-                const uint32_t row = (uint32_t)((m0 + r) * p.lda_bytes) + aofs + (uint32_t)pl * (uint32_t)p.a_plane_bytes + kofs;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, LDS_AS(st + (pl * BM + r) * KTILE_BYTES), 16,
-                                                         voff_a[(r >> 3) & 1] + row, 0, 0, 0);
+                uint32_t ofs;
+                if constexpr (CONV)
+                    ofs = pix[j] + tofs;
+                else
+                    ofs = voff_a[(r >> 3) & 1] + ((uint32_t)((m0 + r) * p.lda_bytes) + aofs +
+                                                  (uint32_t)pl * (uint32_t)p.a_plane_bytes + kofs);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, LDS_AS(st + (pl * BM + r) * KTILE_BYTES), 16, ofs, 0, 0, 0);
             }
+        if constexpr (CONV) tofs = lane_ofs[(kt + 1) * 8];  // k-tiles are loaded in order
 #pragma unroll
         for (int j = 0; j < IB; ++j) {
             const int r = (j * NW + wave) * 8;
@@ -701,20 +740,24 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
     }
 }
 
-template <int KD, int BM, int BN, int WGM, int WGN, int NS, int RS = 0>
+template <int KD, int BM, int BN, int WGM, int WGN, int NS, int RS = 0, bool CONV = false>
 hipError_t launch_one(const GemmArgs& a, int batch, hipStream_t st) {
     // the grid was sized from the configuration table: it must be exactly this tile's
     if ((int64_t)a.tiles_m * BM < a.M || (int64_t)(a.tiles_m - 1) * BM >= a.M || (int64_t)a.tiles_n * BN < a.N ||
         (int64_t)(a.tiles_n - 1) * BN >= a.N)
         return hipErrorInvalidValue;
     dim3 grid(a.tiles_m * a.tiles_n, batch);
-    typename KernelArgs<KD>::type k;
+    typename KernelArgs<KD, CONV>::type k;
     static_cast<GemmCore&>(k) = a;
+    if constexpr (CONV) {
+        k.conv = a.conv;
+        if ((a.kt + NS + 1) * 8 > CONV_CHUNKS) return hipErrorInvalidValue;
+    }
     if constexpr (KD == KIND_I8)
         k.qepi = a.qepi;
     else
         k.epi = a.epi;
-    hipLaunchKernelGGL((gemm_kernel<KD, BM, BN, WGM, WGN, NS, RS>), grid, dim3(64 * WGM * WGN), 0, st, k);
+    hipLaunchKernelGGL((gemm_kernel<KD, BM, BN, WGM, WGN, NS, RS, CONV>), grid, dim3(64 * WGM * WGN), 0, st, k);
     return hipGetLastError();
 }
 
@@ -725,5 +768,6 @@ hipError_t launch_gemm_bf16(int cfg, const GemmArgs& a, int batch, hipStream_t s
 hipError_t launch_gemm_bf16x2(int cfg, const GemmArgs& a, int batch, hipStream_t st);
 hipError_t launch_gemm_f32(int cfg, const GemmArgs& a, int batch, hipStream_t st);
 hipError_t launch_gemm_i8(int cfg, const GemmArgs& a, int batch, hipStream_t st);
+hipError_t launch_gemm_i8_conv(int cfg, const GemmArgs& a, int batch, hipStream_t st);
 
 }  // namespace ingot

@@ -39,18 +39,38 @@ struct GemmCore {
     int64_t ldy;
 };
 
+// The A rows of an int8 product taken from a convolution's activations, which
+// lie [image][padded row][padded column][group][channel] with the padding in
+// place and each group's channels padded to whole 16-byte chunks: row m is
+// output pixel m % p of image m / p, and its k runs over the taps, each tap's
+// channels (cpc chunks) together.
+struct ConvRows {
+    int cpc;        // 16-byte chunks of channels per tap and group (0: A is a matrix)
+    int taps, kw;   // taps of the kernel, taps of a kernel row
+    int p, ow;      // output pixels of an image, of a row
+    int img_bytes, oh_bytes, ow_bytes;  // between images, output rows, output columns
+    int kh_bytes, kw_bytes;             // between kernel rows, taps of a row
+};
+// Chunk offsets a workgroup's table holds (taps · cpc rounded to k-tiles, plus
+// the k-tiles past the end that the pipeline asks for).
+constexpr int CONV_CHUNKS = 1536;
+
 // What the host fills; a launch passes the kernel only the epilogue its kind
 // reads (GemmArgsF or GemmArgsQ): the host cost of a launch grows with the
 // size of its arguments.
 struct GemmArgs : GemmCore {
     Epi epi;
     QEpi qepi;
+    ConvRows conv;
 };
 struct GemmArgsF : GemmCore {
     Epi epi;
 };
 struct GemmArgsQ : GemmCore {
     QEpi qepi;
+};
+struct GemmArgsConv : GemmArgsQ {
+    ConvRows conv;
 };
 
 struct GemmConfig {
@@ -157,6 +177,13 @@ struct QconvGeom {
 // Groups are col_group bytes apart; kgl is a multiple of 16.
 hipError_t launch_qim2col(const void* x, const QconvGeom& g, int rows, int kg, int kgl, uint8_t pad, void* col,
                           int64_t col_group, hipStream_t st);
+// The operands of the pixel GEMM (ConvRows), in one launch: x of `images` images
+// as [image][hp][wp][G][cgp] signed bytes (u8 x less 128; pad outside the image
+// and past a group's channels) and the packed weight (rows ldw bytes apart, k =
+// channel, tap) as rows of taps · cgp bytes, k = tap, channel (zero past a
+// group's channels), ldp bytes apart.
+hipError_t launch_qconv_layout(const void* x, const QconvGeom& g, int images, int hp, int wp, int cgp, uint8_t pad,
+                               int x_u8, void* xt, const int8_t* w, int64_t ldw, int64_t ldp, int8_t* wt, hipStream_t st);
 // Direct QLinearConv of every output element (weight rows ldw bytes apart).
 hipError_t launch_qconv_direct(const void* x, int x_u8, const QconvGeom& g, const int8_t* w, int64_t ldw,
                                const int32_t* bias, const float* mult, int32_t zx, float zy, int y_u8, void* y,

@@ -2,13 +2,18 @@
 //
 // Two routes, both exact in int32 and requantised with the reference's
 // expression (vek.RequantU8/I8, kernels/vek/quant_amd64.go:52-70):
-//  * im2col → int8 GEMM: qim2col_kernel writes, per group, the byte column
-//    matrix col[row = image·P + pixel][k = (c, kh, kw)] of the raw activations
-//    (u8 or s8, taps outside the image hold the zero point zx, k past the
-//    group's K zero) in whole 128-byte k-tiles, the A operand of the int8 MFMA
-//    GEMM; its epilogue adds −zx′·ΣW + bias per output channel, requantises
-//    with that channel's multiplier and stores the NCHW planes. The
-//    reference's pointwise and im2colTiled paths (:612-673) are this route.
+//  * pixel GEMM: one launch writes the activations channel-innermost with
+//    their padding (the zero point) and the weight with the taps outermost;
+//    the int8 MFMA GEMM then reads its A rows, the output pixels, straight from
+//    those activations (gemm_kernel's CONV), adds −zx′·ΣW + bias per output
+//    channel, requantises with that channel's multiplier and stores the NCHW
+//    planes. The reference's pointwise and im2colTiled paths (:612-673).
+//  * im2col → int8 GEMM, for reductions longer than the pixel GEMM's chunk
+//    table and for groups so narrow that padding a tap's channels to 16 would
+//    lengthen them: qim2col_kernel writes, per group, the byte column matrix
+//    col[row = image·P + pixel][k = (c, kh, kw)] of the raw activations (taps
+//    outside the image hold the zero point zx, k past the group's K zero) in
+//    whole 128-byte k-tiles, the A operand of the same GEMM.
 //  * depthwise: v_dot4 over a kernel row; 3 × 3 and 5 × 5 kernels of stride 1
 //    or 2 by lanes that each own 4 × 4 outputs and read their rows straight
 //    from memory, other forms by a wave per strip of one output plane, the
@@ -37,6 +42,118 @@ __device__ __forceinline__ uint8_t requant_byte(int32_t v, float mult, float zy,
     const int iv = u8 ? (r <= 0.f ? 0 : (r >= 255.f ? 255 : (int)r))
                       : (r <= -128.f ? -128 : (r >= 127.f ? 127 : (int)r));
     return (uint8_t)iv;
+}
+
+// 4 bytes of an image row from column c on, columns outside [0, w) holding pad:
+// one load at the nearest place inside the row, moved into position (w >= 4).
+struct RowWord {
+    int off, up;    // where to load; bytes to move the word up (> 0) or down
+    uint32_t keep;  // the bytes that lie inside
+    __device__ __forceinline__ RowWord(int c, int w) {
+        off = min(max(c, 0), w - 4);
+        up = off - c;
+        keep = up > 3 || up < -3 ? 0u : (up >= 0 ? ~0u << (8 * up) : ~0u >> (-8 * up));
+    }
+    __device__ __forceinline__ uint32_t place(uint32_t raw, uint32_t pad) const {
+        const uint32_t v = up >= 0 ? raw << (8 * (up & 3)) : raw >> (8 * (-up & 3));
+        return (v & keep) | (pad & ~keep);
+    }
+};
+
+// Operands of the pixel GEMM. Workgroups below x_blocks move 64 channels × 64
+// columns of one padded row: each thread loads 4 columns of 4 channels,
+// transposes them with byte permutes, and the tile passes through LDS so that
+// the stores are 16 channels of a pixel. The others move 16-byte chunks of the
+// weight, neighbouring threads on the taps of one channel run.
+struct QlayoutArgs {
+    const uint8_t* x;
+    uint8_t* xt;
+    const int8_t* w;
+    int8_t* wt;
+    QconvGeom g;
+    int hp, wp, cgp;       // padded rows, columns; channels of a group rounded to 16
+    int ctiles, wtiles;    // 64-wide tiles over the channels of all groups (padded), over wp
+    int64_t x_blocks, w_chunks;
+    int64_t ldw, ldp;
+    uint32_t pad;          // the zero point in every byte
+    uint32_t flip;         // 0x80808080: u8 → s8
+};
+
+__global__ void __launch_bounds__(256) qconv_layout_kernel(QlayoutArgs p) {
+    const QconvGeom& g = p.g;
+    const int tid = threadIdx.x;
+    if (blockIdx.x >= p.x_blocks) {
+        const int64_t i = (blockIdx.x - p.x_blocks) * 256 + tid;
+        if (i >= p.w_chunks) return;
+        const int taps = g.KH * g.KW, cpc = p.cgp >> 4;
+        const int64_t run = i / taps;  // (output channel, chunk of 16 input channels)
+        const int tap = (int)(i - run * taps), m = (int)(run / cpc), cb = (int)(run - (int64_t)m * cpc);
+        const int8_t* src = p.w + (int64_t)m * p.ldw + (int64_t)cb * 16 * taps + tap;
+        int8_t v[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = cb * 16 + e < g.Cg ? src[(int64_t)e * taps] : (int8_t)0;
+        i32x4_t o;
+        __builtin_memcpy(&o, v, 16);
+        *(i32x4_t*)(p.wt + (int64_t)m * p.ldp + (int64_t)tap * p.cgp + cb * 16) = o;
+        return;
+    }
+    constexpr int PITCH = 17;  // words of a pixel's 64 channels, odd
+    __shared__ uint32_t tile[64 * PITCH];
+    uint32_t b = blockIdx.x;
+    const int ct = (int)(b % p.ctiles);
+    b /= p.ctiles;
+    const int wt = (int)(b % p.wtiles);
+    b /= p.wtiles;
+    const int ih = (int)(b % p.hp) - g.pt;  // input row (outside: padding)
+    const int64_t row = b;                   // image · hp + padded row
+    const int img = (int)(b / p.hp);
+    const int cq = tid >> 4, pq = tid & 15;  // 4 channels, 4 columns
+    const int c0 = ct * 64 + cq * 4;         // channel in the padded order: group · cgp + channel
+    const int col = wt * 64 + pq * 4 - g.pl;
+    uint32_t v[4];
+    if (ih < 0 || ih >= g.H) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = p.pad;
+    } else {
+        const int grp = c0 / p.cgp, cin = c0 - grp * p.cgp;  // 4 channels never straddle groups (cgp % 16 == 0)
+        const uint8_t* src = p.x + (((int64_t)img * g.C + (int64_t)grp * g.Cg + cin) * g.H + ih) * g.W;
+        const int64_t plane = (int64_t)g.H * g.W;
+        const int have = grp < g.G ? g.Cg - cin : 0;
+        if (g.W >= 4) {
+            const RowWord rw(col, g.W);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = p.pad;
+                if (e < have) __builtin_memcpy(&v[e], src + e * plane + rw.off, 4);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = rw.place(v[e], p.pad);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = p.pad;
+                for (int i = 0; i < 4; ++i)
+                    if (e < have && col + i >= 0 && col + i < g.W)
+                        v[e] = (v[e] & ~(0xFFu << (8 * i))) | ((uint32_t)src[e * plane + col + i] << (8 * i));
+            }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] ^= p.flip;
+    // 4 channels × 4 columns → one word of 4 channels per column
+    const uint32_t lo01 = __builtin_amdgcn_perm(v[1], v[0], 0x05010400), hi01 = __builtin_amdgcn_perm(v[1], v[0], 0x07030602);
+    const uint32_t lo23 = __builtin_amdgcn_perm(v[3], v[2], 0x05010400), hi23 = __builtin_amdgcn_perm(v[3], v[2], 0x07030602);
+    tile[(pq * 4 + 0) * PITCH + cq] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100);
+    tile[(pq * 4 + 1) * PITCH + cq] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302);
+    tile[(pq * 4 + 2) * PITCH + cq] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100);
+    tile[(pq * 4 + 3) * PITCH + cq] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302);
+    __syncthreads();
+    const int px = tid >> 2, cc = tid & 3;  // one 16-byte chunk per thread
+    const int64_t pitch = (int64_t)g.G * p.cgp;
+    if (wt * 64 + px < p.wp && ct * 64 + cc * 16 < pitch) {
+        const uint32_t* t = tile + px * PITCH + cc * 4;
+        *(uint4*)(p.xt + (row * p.wp + wt * 64 + px) * pitch + ct * 64 + cc * 16) = make_uint4(t[0], t[1], t[2], t[3]);
+    }
 }
 
 // One thread writes 16 consecutive k of one row (a 16-byte store); a row is
@@ -486,6 +603,23 @@ hipError_t launch_qim2col(const void* x, const QconvGeom& g, int rows, int kg, i
     const int64_t blocks = (threads + 255) / 256;
     hipLaunchKernelGGL(qim2col_kernel, dim3((unsigned)blocks, (unsigned)g.G), dim3(256), 0, st, (const uint8_t*)x, g,
                        rows, kg, kgl, pad, (uint8_t*)col, col_group);
+    return hipGetLastError();
+}
+
+hipError_t launch_qconv_layout(const void* x, const QconvGeom& g, int images, int hp, int wp, int cgp, uint8_t pad,
+                               int x_u8, void* xt, const int8_t* w, int64_t ldw, int64_t ldp, int8_t* wt, hipStream_t st) {
+    QlayoutArgs p;
+    p.x = (const uint8_t*)x, p.xt = (uint8_t*)xt, p.w = w, p.wt = wt, p.g = g;
+    p.hp = hp, p.wp = wp, p.cgp = cgp, p.ldw = ldw, p.ldp = ldp;
+    p.ctiles = (g.G * cgp + 63) / 64;
+    p.wtiles = (wp + 63) / 64;
+    p.x_blocks = (int64_t)images * hp * p.wtiles * p.ctiles;
+    p.w_chunks = (int64_t)g.M * g.KH * g.KW * (cgp / 16);
+    p.pad = pad * 0x01010101u;
+    p.flip = x_u8 ? 0x80808080u : 0u;
+    const int64_t blocks = p.x_blocks + (p.w_chunks + 255) / 256;
+    if (blocks >= (1 << 24)) return hipErrorInvalidValue;  // 256 threads each: the grid stays below 2^32
+    hipLaunchKernelGGL(qconv_layout_kernel, dim3((unsigned)blocks), dim3(256), 0, st, p);
     return hipGetLastError();
 }
 

@@ -938,12 +938,16 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
     g.dh = (int)a->dilation_h, g.dw = (int)a->dilation_w, g.pt = (int)a->pad_top, g.pl = (int)a->pad_left;
     g.OH = (int)OH, g.OW = (int)OW;
     const int yu8 = a->y_dtype == INGOT_DT_U8 ? 1 : 0;
-    // Route: a GEMM needs output-channel and reduction width to fill MFMA
-    // tiles; depthwise and narrow groups run direct. INGOT_QCONV_PATH=1/2
-    // forces direct/GEMM (tests run both routes on the same cases).
+    // Route: a GEMM needs output channels to fill MFMA tiles; depthwise and
+    // narrow groups run direct, and so do short reductions of few outputs, where
+    // one launch beats the layout and the GEMM (on MI355X, kernels alone, direct /
+    // GEMM: 4 × 128 × 28 × 28 outputs of K = 3 5.7 / 7.4 µs, of K = 19 12.4 / 8.0;
+    // 8 × 32 × 32 × 32 of K = 27 9.2 / 8.1: the line is 2^22 products).
+    // INGOT_QCONV_PATH=1/2/3 forces direct / pixel GEMM / im2col GEMM (tests run
+    // the routes on the same cases).
     const int path = s->qconv_path;
     const int64_t kgl = round_up(K, 128);
-    const bool gemm = path == 2 || (path != 1 && Mg >= 16 && K >= 32);
+    const bool gemm = path >= 2 || (path != 1 && Mg >= 16 && (K >= 32 || total * K >= (1ll << 22)));
     if (!gemm) {
         if (path != 1) {
             bool done = false;
@@ -957,20 +961,95 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
         if (e != hipSuccess) return hip_fail(e, "qconv direct");
         return INGOT_OK;
     }
+    if ((P + 256) * kgl >= lim || (w->np + 256) * w->ldk >= lim)
+        return fail(INGOT_EDECLINED, "qlinear_conv: column matrix or weight larger than 2 GiB");
+    GemmArgs ga;
+    memset(&ga, 0, sizeof ga);
+    ga.N = (int)Mg;
+    ga.stride_y = Mg * P;
+    ga.ldy = Mg;
+    ga.qepi.colsum = w->colsum;
+    ga.qepi.neg_za = (int32_t)(0u - (uint32_t)(u8 ? a->zx - 128 : a->zx));
+    ga.qepi.yq_u8 = yu8;
+    ga.qepi.rq_zy = (float)a->zy;
+    ga.qepi.rq_mults = a->d_mult;
+    ga.qepi.bias = a->d_bias;
+    ga.qepi.col_batch = (int32_t)Mg;
+    ga.qepi.conv_p = (int32_t)P;
+    ga.qepi.conv_img = a->m * P;
+    const GemmConfig* cf;
+    gemm_configs(KIND_I8, &cf);
+    const auto run_rows = [&](int64_t rows) {
+        ga.M = (int)rows;
+        const int cfg = pick_config(KIND_I8, rows, Mg, a->group, s->num_cus, s->force_gemm_cfg);
+        ga.tiles_m = (int)((rows + cf[cfg].bm - 1) / cf[cfg].bm);
+        ga.tiles_n = (int)((Mg + cf[cfg].bn - 1) / cf[cfg].bn);
+        return launch_gemm(KIND_I8, cfg, ga, (int)a->group, s->stream);
+    };
+
+    // Pixel GEMM: the padded channel-innermost copy of x in place of the column
+    // matrix, which repeats every input byte once per tap (1 × 256 × 56 × 56 →
+    // 256, 3 × 3, on MI355X: im2col 24.3 + GEMM 12.6 µs; layout 4.0 + GEMM 10.2).
+    const int64_t taps = a->kh * a->kw, cgp = round_up(Cg, 16), kt_px = (taps * cgp + 127) / 128;
+    const int64_t hp = (OH - 1) * a->stride_h + (a->kh - 1) * a->dilation_h + 1;
+    const int64_t wp = (OW - 1) * a->stride_w + (a->kw - 1) * a->dilation_w + 1;
+    const int64_t px_bytes = a->group * cgp, ldp = kt_px * 128 + 128;
+    if (path != 3 && (kt_px + 6) * 8 <= CONV_CHUNKS && hp * wp < ((int64_t)1 << 30) / px_bytes &&
+        (a->m + 256) * ldp < ((int64_t)1 << 30)) {
+        const int64_t img_bytes = hp * wp * px_bytes;
+        const int64_t tiles = hp * ((wp + 63) / 64) * ((px_bytes + 63) / 64);  // of the layout launch, per image
+        const int64_t ipc = std::max<int64_t>(
+            1, std::min({(int64_t)a->n, ((int64_t)512 << 20) / img_bytes, ((int64_t)1 << 22) / tiles}));
+        if (tiles < ((int64_t)1 << 23)) {
+            const int64_t xt_bytes = round_up(ipc * img_bytes, 256);
+            void* ws;
+            rc = ws_reserve(s, (size_t)(xt_bytes + a->m * ldp), &ws);
+            if (rc) return rc;
+            int8_t* wt = (int8_t*)ws + xt_bytes;
+            ga.a = (const char*)ws;
+            ga.stride_a_bytes = cgp;
+            ga.b = (const char*)wt;
+            ga.ldb_bytes = ldp;
+            ga.stride_b_bytes = a->group > 1 ? Mg * ldp : 0;
+            ga.b_bytes = (uint32_t)((Mg - 1) * ldp + kt_px * 128);
+            ga.b_rows = (int)Mg;
+            ga.kt = (int)kt_px;
+            ga.conv = {(int)(cgp / 16), (int)taps, (int)a->kw, (int)P, (int)OW, (int)img_bytes,
+                       (int)(a->stride_h * wp * px_bytes), (int)(a->stride_w * px_bytes),
+                       (int)(a->dilation_h * wp * px_bytes), (int)(a->dilation_w * px_bytes)};
+            for (int64_t n0 = 0; n0 < a->n; n0 += ipc) {
+                const int64_t imgs = std::min(ipc, a->n - n0);
+                hipError_t e = launch_qconv_layout((const uint8_t*)a->d_x + n0 * a->c * a->h * a->w, g, (int)imgs, (int)hp,
+                                                   (int)wp, (int)cgp, (uint8_t)a->zx, u8 ? 1 : 0, ws,
+                                                   (const int8_t*)w->data, w->ldk, ldp, wt, s->stream);
+                if (e != hipSuccess) return hip_fail(e, "qconv layout");
+                ga.a_bytes = (uint32_t)(imgs * img_bytes - (a->group - 1) * cgp);
+                ga.qepi.yq = (uint8_t*)a->d_y + n0 * a->m * P;
+                e = run_rows(imgs * P);
+                if (e != hipSuccess) return hip_fail(e, "qconv gemm");
+            }
+            return INGOT_OK;
+        }
+    }
+
     // Images per chunk: the column matrix of one chunk stays under ~512 MiB
     // and each group's rows under the 2 GiB buffer-offset limit.
     const int64_t per_img = P * kgl;
-    if ((P + 256) * kgl >= lim || (w->np + 256) * w->ldk >= lim)
-        return fail(INGOT_EDECLINED, "qlinear_conv: column matrix or weight larger than 2 GiB");
     int64_t ipc = std::max<int64_t>(1, ((int64_t)512 << 20) / (a->group * per_img));
     ipc = std::min(ipc, std::max<int64_t>(1, (lim - 256 * kgl) / per_img - 1));
     ipc = std::min(ipc, a->n);
     void* ws;
     rc = ws_reserve(s, (size_t)(a->group * ipc * per_img), &ws);
     if (rc) return rc;
-    const int cfg0 = pick_config(KIND_I8, ipc * P, Mg, a->group, s->num_cus, s->force_gemm_cfg);
-    const GemmConfig* cf;
-    gemm_configs(KIND_I8, &cf);
+    ga.a = (const char*)ws;
+    ga.lda_bytes = kgl;
+    ga.a_xor = u8 ? 1 : 0;
+    ga.b = (const char*)w->data;
+    ga.ldb_bytes = w->ldk;
+    ga.stride_b_bytes = a->group > 1 ? Mg * w->ldk : 0;
+    ga.b_bytes = (uint32_t)(a->group > 1 ? Mg * w->ldk : w->np * w->ldk);
+    ga.b_rows = (int)w->np;
+    ga.kt = (int)(kgl / KTILE_BYTES);
     for (int64_t n0 = 0; n0 < a->n; n0 += ipc) {
         const int64_t imgs = std::min(ipc, a->n - n0);
         const int64_t rows = imgs * P;
@@ -978,37 +1057,10 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
         hipError_t e = launch_qim2col((const uint8_t*)a->d_x + n0 * a->c * a->h * a->w, g, (int)rows, (int)K,
                                       (int)kgl, (uint8_t)a->zx, ws, col_group, s->stream);
         if (e != hipSuccess) return hip_fail(e, "qim2col");
-        GemmArgs ga;
-        memset(&ga, 0, sizeof ga);
-        ga.a = (const char*)ws;
-        ga.lda_bytes = kgl;
         ga.stride_a_bytes = col_group;
         ga.a_bytes = (uint32_t)col_group;
-        ga.a_xor = u8 ? 1 : 0;
-        ga.b = (const char*)w->data;
-        ga.ldb_bytes = w->ldk;
-        ga.stride_b_bytes = a->group > 1 ? Mg * w->ldk : 0;
-        ga.b_bytes = (uint32_t)(a->group > 1 ? Mg * w->ldk : w->np * w->ldk);
-        ga.b_rows = (int)w->np;
-        ga.M = (int)rows;
-        ga.N = (int)Mg;
-        ga.kt = (int)(kgl / KTILE_BYTES);
-        ga.stride_y = Mg * P;
-        ga.ldy = Mg;
-        ga.qepi.colsum = w->colsum;
-        ga.qepi.neg_za = (int32_t)(0u - (uint32_t)(u8 ? a->zx - 128 : a->zx));
         ga.qepi.yq = (uint8_t*)a->d_y + n0 * a->m * P;
-        ga.qepi.yq_u8 = yu8;
-        ga.qepi.rq_zy = (float)a->zy;
-        ga.qepi.rq_mults = a->d_mult;
-        ga.qepi.bias = a->d_bias;
-        ga.qepi.col_batch = (int32_t)Mg;
-        ga.qepi.conv_p = (int32_t)P;
-        ga.qepi.conv_img = a->m * P;
-        const int cfg = rows == ipc * P ? cfg0 : pick_config(KIND_I8, rows, Mg, a->group, s->num_cus, s->force_gemm_cfg);
-        ga.tiles_m = (int)((rows + cf[cfg].bm - 1) / cf[cfg].bm);
-        ga.tiles_n = (int)((Mg + cf[cfg].bn - 1) / cf[cfg].bn);
-        e = launch_gemm(KIND_I8, cfg, ga, (int)a->group, s->stream);
+        e = run_rows(rows);
         if (e != hipSuccess) return hip_fail(e, "qconv gemm");
     }
     return INGOT_OK;

@@ -172,6 +172,36 @@ def test_depthwise_strips(sess, case):
         np.testing.assert_array_equal(got, oracle.qlinear_conv(x, zx, wt, bias, mult, zy, y_u8, **kw_))
 
 
+# Pixel GEMM: channels around whole 16-byte chunks, images narrower than a word and wider than a tile, groups whose
+# channels pad, pads past the image, strides that skip columns, several images, a reduction of many k-tiles and one past
+# the chunk table (which falls back to im2col).
+PIXEL_CASES = [
+    # n, c, h, w, m, kh, kw, g, strides, dilations, pads
+    (2, 16, 9, 3, 17, 3, 3, 1, (1, 1), (1, 1), (1, 1, 1, 1)),
+    (1, 15, 5, 2, 16, 3, 2, 1, (1, 1), (1, 1), (1, 0, 1, 2)),
+    (3, 17, 6, 1, 33, 3, 1, 1, (2, 1), (1, 1), (1, 0, 1, 0)),
+    (2, 51, 7, 130, 21, 1, 3, 3, (1, 2), (1, 1), (0, 1, 0, 1)),
+    (1, 64, 8, 70, 64, 3, 3, 2, (1, 1), (2, 2), (4, 5, 2, 3)),
+    (2, 33, 12, 65, 40, 1, 1, 1, (2, 2), (1, 1), (0, 0, 0, 0)),
+    (1, 700, 5, 6, 24, 3, 3, 1, (1, 1), (1, 1), (1, 1, 1, 1)),
+    (1, 2700, 3, 4, 16, 3, 3, 1, (1, 1), (1, 1), (1, 1, 1, 1)),
+]
+
+
+@pytest.mark.parametrize("path", [2, 3])
+@pytest.mark.parametrize("case", PIXEL_CASES, ids=[f"p{i}" for i in range(len(PIXEL_CASES))])
+def test_pixel_gemm(env_session, path, case):
+    n, c, h, w, m, kh, kw, g, st, dl, pads = case
+    announce(f"qconv pixel gemm {case} path={path}")
+    rng = np.random.default_rng(sum(case[:7]))
+    qs = env_session(INGOT_QCONV_PATH=path)
+    for x_dtype, zx, y_u8, zy, with_bias in [(np.uint8, 131, True, 9, True), (np.int8, -128, False, -5, False)]:
+        x, zx, wt, bias, mult, *_ = make_case(rng, n, c, h, w, m, kh, kw, g, x_dtype, zx, with_bias)
+        kw_ = dict(group=g, strides=st, dilations=dl, pads=pads)
+        got = run_conv(qs, x, zx, wt, bias, mult, zy, y_u8, **kw_)
+        np.testing.assert_array_equal(got, oracle.qlinear_conv(x, zx, wt, bias, mult, zy, y_u8, **kw_))
+
+
 def test_empty_and_degenerate(sess):
     announce("qconv empty")
     rng = np.random.default_rng(0)
