@@ -278,6 +278,52 @@ def test_dequantize_linear_op(sess):
         op.run(dev(sess, x, L.DT_I32), dev(sess, np.ones(5, np.float32)))
 
 
+@pytest.mark.parametrize("n,n_scale,inner", [(1, 1, 1), (1023, 1, 1), (4099, 1, 7), (3 * 5, 5, 1), (70 * 257, 257, 1),
+                                             (6 * 4 * 3, 4, 3), (2 * 3 * 1030, 3, 1030), (2 * 9 * 64 + 17, 9, 64),
+                                             (3 * 5 - 2, 5, 1)])
+@pytest.mark.parametrize("dtype", [np.uint8, np.int8, np.int32])
+def test_dequantize_views(sess, n, n_scale, inner, dtype):
+    """Per-tensor, per-column and per-row scales at widths around 4 elements and a thread row, with row tails and
+    unaligned starts, zero points of one or every scale: exactly the oracle's values (whole numbers below 2^24 and
+    one rounded product)."""
+    announce(f"dequant n={n} scales={n_scale} inner={inner} {np.dtype(dtype).name}")
+    rng = np.random.default_rng(n + n_scale)
+    info = np.iinfo(dtype)
+    x = rng.integers(max(info.min, -100000), min(info.max, 100000) + 1, n).astype(dtype)
+    sc = rng.uniform(0.01, 0.1, n_scale).astype(np.float32)
+    code = {np.uint8: L.DT_U8, np.int8: L.DT_I8, np.int32: L.DT_I32}[dtype]
+    for zp in (None, rng.integers(0, 100, 1).astype(np.int8), rng.integers(-100, 100, n_scale).astype(np.int32)):
+        y = sess.empty(L.DT_F32, (n,))
+        dz = None if zp is None else dev(sess, zp, L.DT_I8 if zp.dtype == np.int8 else L.DT_I32)
+        sess.dequantize_linear(dev(sess, x, code), dev(sess, sc), y, inner=inner, zp=dz)
+        np.testing.assert_array_equal(y.numpy(), oracle.dequantize_linear(x, sc, inner=inner, zp=zp))
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (1, 1027), (5, 3), (9, 257), (33, 1028)])
+def test_activation_bias_views(sess, rows, cols):
+    """The bias row at widths around 4 elements and a thread row (x + bias is one rounded sum; ReLU is exact), the
+    same pass without a bias, the bf16 cast and a fill of bytes at odd starts and lengths."""
+    announce(f"activation bias {rows}x{cols}")
+    rng = np.random.default_rng(rows * cols)
+    x = rng.normal(0, 1, (rows, cols)).astype(np.float32)
+    b = rng.normal(0, 1, cols).astype(np.float32)
+    dx, y = dev(sess, x), sess.empty(L.DT_F32, (rows, cols))
+    sess.activation(dx, y, rows, cols, L.ACT_RELU, bias=dev(sess, b))
+    np.testing.assert_array_equal(y.numpy(), np.maximum(x + b, 0))
+    sess.activation(dx, y, rows, cols, L.ACT_RELU)
+    np.testing.assert_array_equal(y.numpy(), np.maximum(x, 0))
+    h = sess.empty(L.DT_BF16, (rows, cols))
+    sess.cast_bf16(dx, h)
+    np.testing.assert_array_equal(h.numpy(), oracle.f32_to_bf16(x))
+    buf = dev(sess, np.zeros(rows * cols + 64, np.uint8), L.DT_U8)
+    for start, count in ((0, rows * cols + 64), (3, rows * cols + 2), (13, 1), (1, 31)):
+        sess.memset(buf, 0)
+        L.check(sess.lib.ingot_rocm_memset(sess.h, buf.ptr + start, 0xA5, count))
+        want = np.zeros(rows * cols + 64, np.uint8)
+        want[start:start + count] = 0xA5
+        np.testing.assert_array_equal(buf.numpy(), want)
+
+
 @pytest.mark.parametrize("name,domain,attrs,code", [("Relu", "", {}, L.ACT_RELU), ("Gelu", "ingot", {}, L.ACT_GELU_ERF),
                                                    ("Gelu", "", {"approximate": "tanh"}, L.ACT_GELU_TANH),
                                                    ("Sigmoid", "", {}, L.ACT_SIGMOID)])
