@@ -67,14 +67,10 @@ __device__ __forceinline__ void mma16<KIND_BF16X2>(f32x4_t& acc, const i32x4_t& 
     mma16<KIND_BF16>(acc, x, y);
 }
 
-template <>
-__device__ __forceinline__ void mma16<KIND_F32>(f32x4_t& acc, const i32x4_t& x, const i32x4_t& y) {
-    const f32x4_t xf = __builtin_bit_cast(f32x4_t, x);
-    const f32x4_t yf = __builtin_bit_cast(f32x4_t, y);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xf[0], yf[0], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xf[1], yf[1], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xf[2], yf[2], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xf[3], yf[3], acc, 0, 0, 0);
+// One of the four steps of a 16-byte chunk of f32.
+__device__ __forceinline__ void mma16_f32(f32x4_t& acc, const i32x4_t& x, const i32x4_t& y, int e) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(f32x4_t, x)[e], __builtin_bit_cast(f32x4_t, y)[e], acc, 0,
+                                               0, 0);
 }
 
 template <>
@@ -402,12 +398,27 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
     auto read_frags = [&](const char* st, int s, FragA& fa, FragB& fb) {
         read_frags2(st, st + AP * BM * KTILE_BYTES, s, fa, fb);
     };
-    // the products of one activation plane and one half k-tile
+    // The products of one activation plane and one half k-tile. f32: a chunk
+    // takes four MFMAs on one accumulator, and one that waits for its
+    // predecessor's result loses issue slots (with one wave per SIMD nothing else
+    // fills them), so each step runs over all accumulators before the next;
+    // an accumulator still sees its steps in order (on MI355X 1024 × 768 → 3072
+    // 40.1 → 39.2 µs, 3072 → 768 with 32×96 tiles unchanged, 2048 × 2048 → 4096
+    // 250 → 244).
     auto mma_plane = [&](const i32x4_t (&fa)[TM], const FragB& fb) {
+        if constexpr (KD == KIND_F32) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) mma16<KD>(acc[i][j], fb[j], fa[i]);
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) mma16_f32(acc[i][j], fb[j], fa[i], e);
+        } else {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) mma16<KD>(acc[i][j], fb[j], fa[i]);
+        }
     };
 
     // Software pipeline over k-tiles: an NS-stage LDS ring filled by DMA NS
