@@ -8,15 +8,16 @@ hipError_t launch_gemm_bf16x2(int cfg, const GemmArgs& a, int batch, hipStream_t
     switch (cfg) {
         case 0: return launch_one<KIND_BF16X2, 256, 256, 4, 2, 2>(a, batch, st);
         case 1: return launch_one<KIND_BF16X2, 256, 192, 4, 2, 2>(a, batch, st);
-        case 2: return launch_one<KIND_BF16X2, 128, 128, 2, 2, 2>(a, batch, st);
-        case 3: return launch_one<KIND_BF16X2, 128, 64, 2, 2, 2>(a, batch, st);
-        case 4: return launch_one<KIND_BF16X2, 64, 64, 2, 2, 2>(a, batch, st);
-        case 5: return launch_one<KIND_BF16X2, 192, 256, 2, 4, 2>(a, batch, st);
-        case 6: return launch_one<KIND_BF16X2, 64, 96, 2, 2, 2>(a, batch, st);
+        case 2: return launch_one<KIND_BF16X2, 128, 128, 4, 2, 3>(a, batch, st);
+        case 3: return launch_one<KIND_BF16X2, 64, 256, 2, 4, 3>(a, batch, st);
+        case 4: return launch_one<KIND_BF16X2, 64, 128, 2, 4, 4>(a, batch, st);
+        case 5: return launch_one<KIND_BF16X2, 32, 64, 2, 2, 4>(a, batch, st);
+        case 6: return launch_one<KIND_BF16X2, 128, 256, 2, 4, 2>(a, batch, st);
         case 7: return launch_one<KIND_BF16X2, 32, 32, 2, 2, 4>(a, batch, st);
         case 8: return launch_one<KIND_BF16X2, 64, 64, 2, 2, 4>(a, batch, st);
         // 256×192 with the weight staged through registers: every load two k-tiles ahead
         case 9: return launch_one<KIND_BF16X2, 256, 192, 4, 2, 2, 2>(a, batch, st);
+        case 10: return launch_one<KIND_BF16X2, 128, 192, 2, 4, 2>(a, batch, st);
     }
     return hipErrorInvalidValue;
 }

@@ -8,18 +8,19 @@ namespace ingot {
 namespace {
 
 // Tile configurations per kind. occupancy: workgroups per CU the LDS and
-// register footprint allow; eff: relative throughput per CU slot (measured
-// on MI355X for the bf16 kernel).
-// Small tiles mostly keep two LDS stages: with several tiles per CU, occupancy
-// (more resident workgroups) hides latency better than a deeper ring. With one
-// tile per CU or fewer (small M, or few columns) each k-tile waits for its own
-// DMA round trip instead, and a four-stage ring pays: the 32×32 and 64×64
-// four-stage entries (bf16 and bf16 hi/lo), measured on MI355X with bf16
-// weights at K = 2048: M = 17–128 × N = 2048–6144 6.5–6.8 µs with 32×32
-// (10.7–11.3 with two-stage 64×64; the hi/lo kind 11.0 vs 35 with 128×128),
-// M = 64 × N = 11264 and M = 256 × N = 6144 11.1 and 15.4 µs with 64×64
-// (18.1 and 18.5 with two stages). Their weights keep the DiT shapes on the
-// large tiles, and they are taken only when every tile is resident at once.
+// register footprint allow. The bf16 kinds' costs are µs per k-tile of a round
+// of tiles that fills the chip, measured on MI355X over M = 16–4096 of the
+// decoder (2048 → 6144, 2048, 11264; 5632 → 2048), encoder (768 ↔ 3072) and
+// diffusion (3072 → 9216, 12288; 12288 → 3072) products, and pick_config adds
+// them up. A k-tile of a small tile costs its LDS traffic and its barrier, not
+// its MFMAs, so what pays is wave tiles that share fragments, eight waves (two
+// per SIMD) and three or four stages: bf16 128×128 0.35–0.43 µs with eight waves
+// and three stages against 0.57 with four waves and two, hi/lo 64×128 0.45–0.50
+// with four stages against 0.67 for two 64×64 tiles of two. Over those products
+// the tiles picked are within 0.1% (bf16) and 0.5% (hi/lo) of the best of 22 and
+// 23 measured, and 8% and 19% faster than the tables they replace (hi/lo, K =
+// 2048: 517 × 6144 42.7 → 35 µs, 1000 × 6144 83 → 48; 517 × 5632 → 2048 75 →
+// 50; bf16 2048 × 12288 → 3072 207 → 139).
 // Entry 9 is entry 1 with the weight staged through registers (gemm_kernel's
 // RS = 2): every load issued two k-tiles ahead instead of one. On MI355X, the
 // DiT MLP-down (M = 4096, N = 3072, K = 12288) right after the MLP-up GEMM
@@ -27,12 +28,32 @@ namespace {
 // 293–294, and after a 1 GiB fill 241 instead of 310; with its operands
 // already cached it is 8–12% slower (249 vs 230 µs), so the runtime takes it
 // only for products whose operands are too large to stay cached.
-// bf16 64×96: at M = 1024, K = 768 (the BERT-size FFN-up and QKV products) two tiles per CU
-// instead of three 64×64 ones: 11.4 vs 12.0–13.1 µs at N = 3072, 10.1 vs 11.5 µs at N = 2304 on
-// MI355X; slower at N = 768 (fewer tiles than CUs), where the weight keeps 64×64 ahead.
-const GemmConfig kBF16Cfgs[] = {{256, 256, 1, 1.00f}, {256, 192, 1, 0.95f, false, 9}, {128, 128, 2, 0.80f}, {128, 64, 3, 0.78f},
-                                {64, 64, 4, 0.65f},   {192, 256, 1, 0.95f}, {64, 96, 3, 0.72f}, {32, 32, 4, 0.60f, true},
-                                {64, 64, 2, 1.00f, true}, {256, 192, 1, 0.f}};
+const GemmConfig kBF16Cfgs[] = {{256, 256, 1, 0.f, false, -1, {1.600f}},
+                                {256, 192, 1, 0.f, false, 9, {1.294f}},
+                                {128, 128, 1, 0.f, false, -1, {0.435f}},
+                                {192, 128, 1, 0.f, false, -1, {0.633f}},
+                                {64, 128, 1, 0.f, false, -1, {0.251f}},
+                                {32, 64, 3, 0.f, false, -1, {0.141f, 0.280f, 0.381f}},
+                                {128, 256, 1, 0.f, false, -1, {0.913f}},
+                                {32, 32, 3, 0.f, false, -1, {0.124f, 0.166f, 0.264f}},
+                                {64, 64, 2, 0.f, false, -1, {0.190f, 0.351f}},
+                                {256, 192, 1, 0.f, false},
+                                {128, 192, 1, 0.f, false, -1, {0.709f}},
+                                {192, 192, 1, 0.f, false, -1, {0.911f}}};
+// hi/lo: tiles of 128 rows hold both activation planes in a stage, which costs
+// fewer operand bytes than the taller tiles' second pass over the weight (1.28
+// against 2.56 µs for 128×192 and 256×192, half the area).
+const GemmConfig kBF16X2Cfgs[] = {{256, 256, 1, 0.f, false, -1, {3.110f}},
+                                  {256, 192, 1, 0.f, false, 9, {2.560f}},
+                                  {128, 128, 1, 0.f, false, -1, {0.812f}},
+                                  {64, 256, 1, 0.f, false, -1, {0.897f}},
+                                  {64, 128, 1, 0.f, false, -1, {0.505f}},
+                                  {32, 64, 2, 0.f, false, -1, {0.229f, 0.423f}},
+                                  {128, 256, 1, 0.f, false, -1, {1.551f}},
+                                  {32, 32, 3, 0.f, false, -1, {0.190f, 0.301f, 0.449f}},
+                                  {64, 64, 1, 0.f, false, -1, {0.373f}},
+                                  {256, 192, 1, 0.f, false},
+                                  {128, 192, 1, 0.f, false, -1, {1.280f}}};
 // f32 32×96: on MI355X 15% faster than 64×64 over the BERT projections (M = 1024;
 // N = 768 gives exactly 256 tiles), slightly slower on ties, so weighted 0.97.
 // 64×96, 64×128, 96×64, 32×128 and 64×192 were no faster on any of them.
@@ -67,8 +88,7 @@ int gemm_configs(GemmKind kind, const GemmConfig** out) {
         case KIND_BF16: *out = kBF16Cfgs; return (int)(sizeof(kBF16Cfgs) / sizeof(kBF16Cfgs[0]));
         case KIND_F32: *out = kF32Cfgs; return (int)(sizeof(kF32Cfgs) / sizeof(kF32Cfgs[0]));
         case KIND_I8: *out = kI8Cfgs; return (int)(sizeof(kI8Cfgs) / sizeof(kI8Cfgs[0]));
-        // the hi/lo kind uses the bf16 kind's tiles (see gemm_kernel for how it runs on them)
-        case KIND_BF16X2: *out = kBF16Cfgs; return (int)(sizeof(kBF16Cfgs) / sizeof(kBF16Cfgs[0]));
+        case KIND_BF16X2: *out = kBF16X2Cfgs; return (int)(sizeof(kBF16X2Cfgs) / sizeof(kBF16X2Cfgs[0]));
         default: break;
     }
     return 0;

@@ -75,10 +75,11 @@ struct GemmArgsConv : GemmArgsQ {
 
 struct GemmConfig {
     int bm, bn;
-    int occupancy;   // workgroups per CU the tile allows (eff 0: never picked by itself)
-    float eff;       // relative per-CU efficiency (tile-size heuristic)
+    int occupancy;   // workgroups per CU the tile allows
+    float eff;       // relative per-CU efficiency (tile-size heuristic of the kinds without costs; 0 and no cost: never picked)
     bool one_round;  // only when every tile is resident at once (a latency-bound shape)
     int deep = -1;   // index of the same tile with loads issued two k-tiles ahead (operands from HBM)
+    float cost[3] = {0, 0, 0};  // measured µs per k-tile with 1, 2, 3 tiles on every CU (0: not measured, eff counts)
 };
 
 // Tile configurations compiled for `kind`; index used by launch_gemm.

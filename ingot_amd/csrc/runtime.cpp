@@ -75,24 +75,38 @@ constexpr int64_t kCacheResidentBytes = (int64_t)128 << 20;
 int ktile_elems(GemmKind k) { return k == KIND_F32 ? 32 : (k == KIND_I8 ? 128 : 64); }
 int kind_size(GemmKind k) { return k == KIND_F32 ? 4 : (k == KIND_I8 || k == KIND_I8G ? 1 : 2); }
 
-// Picks the tile configuration with the least estimated time: full rounds of
-// num_cus·occupancy workgroups, each round as long as the most loaded CU.
-// Deep-ring entries marked one_round apply only when a single round holds
-// every tile. force >= 0 (INGOT_GEMM_CFG) picks that entry when it exists.
-int pick_config(GemmKind kind, int64_t M, int64_t N, int64_t batch, int num_cus, int force) {
+// Picks the tile configuration with the least estimated time. Kinds with
+// measured costs: rounds of num_cus·occupancy tiles, each a fixed 4 µs (launch
+// or refill, prologue, store) plus kt k-tiles at the cost of its most loaded
+// CU; a round that leaves CUs idle runs its tiles up to 30% faster when they are
+// large (64×64 and up: less traffic and power per CU; both numbers from the
+// measurements the costs come from). Other kinds: full rounds weighted by area
+// and eff. Deep-ring entries marked one_round apply only when a single round
+// holds every tile. force >= 0 (INGOT_GEMM_CFG) picks that entry when it exists.
+int pick_config(GemmKind kind, int64_t M, int64_t N, int64_t kt, int64_t batch, int num_cus, int force) {
     const GemmConfig* c;
     const int n = gemm_configs(kind, &c);
     if (force >= 0 && force < n) return force;
     int best = 0;
     double best_t = 1e300;
     for (int i = 0; i < n; ++i) {
-        if (c[i].eff <= 0.f) continue;  // reached only as another entry's deep variant
+        const bool timed = c[i].cost[0] > 0.f;
+        if (!timed && c[i].eff <= 0.f) continue;  // reached only as another entry's deep variant
         const int64_t tiles = ((M + c[i].bm - 1) / c[i].bm) * ((N + c[i].bn - 1) / c[i].bn) * batch;
         const int64_t slots = (int64_t)num_cus * c[i].occupancy;
         const int64_t rounds = (tiles + slots - 1) / slots;
         if (c[i].one_round && rounds > 1) continue;
-        const int64_t per_cu = std::min<int64_t>(c[i].occupancy, (tiles + num_cus - 1) / num_cus);
-        const double t = (double)rounds * (double)per_cu * c[i].bm * c[i].bn / c[i].eff;
+        double t;
+        if (timed) {
+            const int64_t last = tiles - (rounds - 1) * slots;  // 1..slots tiles in the last round
+            const bool large = c[i].bm * c[i].bn >= 64 * 64;
+            const double fill = large && last < num_cus ? 0.7 + 0.3 * (double)last / num_cus : 1.0;
+            t = 4.0 * rounds + kt * ((rounds - 1) * (double)c[i].cost[c[i].occupancy - 1] +
+                                     c[i].cost[(last + num_cus - 1) / num_cus - 1] * fill);
+        } else {
+            const int64_t per_cu = std::min<int64_t>(c[i].occupancy, (tiles + num_cus - 1) / num_cus);
+            t = (double)rounds * (double)per_cu * c[i].bm * c[i].bn / c[i].eff;
+        }
         if (t < best_t * 0.999) {
             best_t = t;
             best = i;
@@ -681,7 +695,7 @@ static int gemm_core(ingot_rocm_session* s, const ingot_rocm_gemm_args* a, const
     g.y = a->d_y;
     g.ldy = a->ldy;
     g.epi = make_epi(a);
-    int cfg = pick_config(kind, a->M, a->N, batch, s->num_cus, s->force_gemm_cfg);
+    int cfg = pick_config(kind, a->M, a->N, g.kt, batch, s->num_cus, s->force_gemm_cfg);
     const GemmConfig* c;
     gemm_configs(kind, &c);
     // Operands larger than half the Infinity Cache (256 MB on MI355X) do not
@@ -868,7 +882,7 @@ static int qgemm(ingot_rocm_session* s, int64_t M, int64_t N, int64_t K, const v
     g.qepi.yq_u8 = yq_u8;
     g.qepi.rq_mult = rq_mult;
     g.qepi.rq_zy = rq_zy;
-    const int cfg = pick_config(KIND_I8, M, N, 1, s->num_cus, s->force_gemm_cfg);
+    const int cfg = pick_config(KIND_I8, M, N, g.kt, 1, s->num_cus, s->force_gemm_cfg);
     const GemmConfig* c;
     gemm_configs(KIND_I8, &c);
     g.tiles_m = (int)((M + c[cfg].bm - 1) / c[cfg].bm);
@@ -981,7 +995,7 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
     gemm_configs(KIND_I8, &cf);
     const auto run_rows = [&](int64_t rows) {
         ga.M = (int)rows;
-        const int cfg = pick_config(KIND_I8, rows, Mg, a->group, s->num_cus, s->force_gemm_cfg);
+        const int cfg = pick_config(KIND_I8, rows, Mg, ga.kt, a->group, s->num_cus, s->force_gemm_cfg);
         ga.tiles_m = (int)((rows + cf[cfg].bm - 1) / cf[cfg].bm);
         ga.tiles_n = (int)((Mg + cf[cfg].bn - 1) / cf[cfg].bn);
         return launch_gemm(KIND_I8, cfg, ga, (int)a->group, s->stream);
