@@ -134,28 +134,34 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p, int txs) {
     }
 }
 
-// Source rows are n-contiguous ([k][n]): 64 × 64 tiles transposed through LDS,
-// so that both the reads (along n) and the writes (16-byte chunks along k) are
-// whole lines. One element a thread, read straight into its padded place, the
-// pack took 18.2 µs for 96 items of 128 × 64 f32 (2.4 MB) on MI355X; with this
-// kernel and the items' own rows only, Q·Kᵀ (read in place) and P·V of 96
-// heads of 128 × 64 went from 48.0 to 19.5 µs together.
+// Source rows are n-contiguous ([k][n]): tiles of 64 n × 64 k (32 k of f32)
+// transposed through LDS, so that both the reads (along n) and the writes
+// (16-byte chunks along k) are whole lines. Bound by its latency at the sizes of
+// attention heads: one element a thread, read straight into its padded place,
+// the pack took 18.2 µs for 96 items of 128 × 64 f32 (2.4 MB) on MI355X, 64 × 64
+// tiles 5.7, 64 × 32 ones (twice the workgroups) 5.1; with this kernel and the
+// items' own rows only, Q·Kᵀ (read in place) and P·V of 96 heads of 128 × 64 went
+// from 48.0 to 19.0 µs together.
+template <typename S>
+constexpr int pack_tk() {
+    return sizeof(S) == 4 ? 32 : 64;
+}
 template <int KD, typename S>
 __global__ __launch_bounds__(256) void pack_cols_kernel(PackArgs p, int64_t tiles, int tiles_k) {
     constexpr int EPC = PackOf<KD>::EPC;
-    constexpr int T = 64;
+    constexpr int T = 64, TK = pack_tk<S>();
     // row pitch in elements: an odd number of 4-byte words
-    constexpr int PITCH = T + (sizeof(S) == 4 ? 1 : (sizeof(S) == 2 ? 2 : 4));
+    constexpr int PITCH = TK + (sizeof(S) == 4 ? 1 : (sizeof(S) == 2 ? 2 : 4));
     __shared__ S tile[T * PITCH];
     const S* src = (const S*)p.src + (int64_t)blockIdx.y * p.src_item;
     char* dst = (char*)p.dst + (int64_t)blockIdx.y * p.dst_item * pack_esz<KD>();
     const int tid = threadIdx.x;
     for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
-        const int64_t j0 = t / tiles_k * T, k0 = t % tiles_k * T;
+        const int64_t j0 = t / tiles_k * T, k0 = t % tiles_k * TK;
         // 4 n of one k per thread and step: 16 threads a source row, 16 rows a step
         const int n4 = (tid & 15) * 4, kr = tid >> 4;
 #pragma unroll
-        for (int i = 0; i < T / 16; ++i) {
+        for (int i = 0; i < TK / 16; ++i) {
             const int kk = kr + i * 16;
             const int64_t have = k0 + kk < p.k ? p.n - (j0 + n4) : 0;
             const S* s = src + (k0 + kk) * p.ld + j0 + n4;
@@ -179,7 +185,7 @@ __global__ __launch_bounds__(256) void pack_cols_kernel(PackArgs p, int64_t tile
             for (int e = 0; e < 4; ++e) tile[(n4 + e) * PITCH + kk] = v[e];
         }
         __syncthreads();
-        constexpr int CPR = T / EPC;  // chunks of a tile row
+        constexpr int CPR = TK / EPC;  // chunks of a tile row
         for (int c = tid; c < T * CPR; c += 256) {
             const int jj = c / CPR, kc = c % CPR * EPC;
             const int64_t j = j0 + jj, k = k0 + kc;
@@ -202,7 +208,7 @@ hipError_t launch_pack(const PackArgs& p, bool rows, int items, hipStream_t st) 
         while (txs < 8 && ((int64_t)PackOf<KD>::EPC << txs) < p.kp) ++txs;
         hipLaunchKernelGGL((pack_rows_kernel<KD, S>), dim3(grid_for(p.np, 256 >> txs), items), dim3(256), 0, st, p, txs);
     } else {
-        const int64_t tiles_k = (p.kp + 63) / 64, tiles = (p.np + 63) / 64 * tiles_k;
+        const int64_t tiles_k = (p.kp + pack_tk<S>() - 1) / pack_tk<S>(), tiles = (p.np + 63) / 64 * tiles_k;
         hipLaunchKernelGGL((pack_cols_kernel<KD, S>), dim3(grid_for(tiles, 1), items), dim3(256), 0, st, p, tiles,
                            (int)tiles_k);
     }
