@@ -8,7 +8,7 @@ namespace ingot {
 namespace {
 
 // Tile configurations per kind. occupancy: workgroups per CU the LDS and
-// register footprint allow. The bf16 kinds' costs are µs per k-tile of a round
+// register footprint allow. The float kinds' costs are µs per k-tile of a round
 // of tiles that fills the chip, measured on MI355X over M = 16–4096 of the
 // decoder (2048 → 6144, 2048, 11264; 5632 → 2048), encoder (768 ↔ 3072) and
 // diffusion (3072 → 9216, 12288; 12288 → 3072) products, and pick_config adds
@@ -54,21 +54,22 @@ const GemmConfig kBF16X2Cfgs[] = {{256, 256, 1, 0.f, false, -1, {3.110f}},
                                   {64, 64, 1, 0.f, false, -1, {0.373f}},
                                   {256, 192, 1, 0.f, false},
                                   {128, 192, 1, 0.f, false, -1, {1.280f}}};
-// f32 32×96: on MI355X 15% faster than 64×64 over the BERT projections (M = 1024;
-// N = 768 gives exactly 256 tiles), slightly slower on ties, so weighted 0.97.
-// 64×96, 64×128, 96×64, 32×128 and 64×192 were no faster on any of them.
-// f32 32×32, four-stage ring: for products with few tiles. The configs[0] Gemm
-// (M = 128, N = 512, K = 256) runs 64 of them instead of 24 32×96 ones: 3.8 vs
-// 6.2 µs per call on MI355X; at M = 32, N = 6144, K = 2048 (64 k-tiles) the ring
-// depth matters: 14.2 µs with four stages, 26.8 with two. 6–12% slower than 32×96
-// on the BERT projections, so weighted 0.8.
-// f32 32×96 with a four-stage ring, when every tile is resident at once (one
-// per CU): the BERT FFN-down (M = 1024, N = 768, K = 3072, 96 k-tiles, one
-// wave per SIMD, so nothing else covers a k-tile's DMA round trip) took 41.6
-// instead of 45.0 µs on MI355X; at three tiles per CU the two-stage ring stays
-// ahead (FFN-up 41.3 vs 43.7), and six stages were slower again (42.1).
-const GemmConfig kF32Cfgs[] = {{128, 128, 2, 0.90f}, {128, 64, 3, 0.95f}, {64, 64, 4, 1.00f}, {32, 96, 4, 0.97f},
-                               {32, 32, 4, 0.80f},   {32, 96, 2, 0.98f, true}};
+// f32: a k-tile is bound by its MFMAs (a tile's area per µs of cost is 7.1–9.0
+// thousand outputs, 9.0 being 147 of the 157 TFLOP/s peak), so the tiles differ
+// little but for how they divide a product over 256 CUs; 32×32 serves products
+// of few tiles (128 × 256 → 512: 64 of them, 3.8 against 6.2 µs with 32×96), the
+// four-stage 32×96 ones of one tile per CU (1024 × 3072 → 768 42.5 against 45.9
+// with two stages), 64×64 and 64×96 with three stages the rest (1024 × 768 →
+// 3072 38.5 against 39.7 µs with two; 260 × 2048 → 4096 50.9 against 55.7 with
+// 32×96; 2048 × 768 → 2304 56.7 against 61). Measured like the bf16 kinds'
+// costs, over M = 16–2048; the picks are within 0.5% of the best of 18 tiles.
+const GemmConfig kF32Cfgs[] = {{128, 128, 2, 0.f, false, -1, {1.816f, 3.670f}},
+                               {128, 64, 3, 0.f, false, -1, {0.936f, 1.826f, 2.750f}},
+                               {64, 64, 3, 0.f, false, -1, {0.484f, 0.924f, 1.368f}},
+                               {32, 96, 3, 0.f, false, -1, {0.432f, 0.755f, 1.229f}},
+                               {32, 32, 3, 0.f, false, -1, {0.169f, 0.294f, 0.429f}},
+                               {32, 96, 2, 0.f, false, -1, {0.387f, 0.740f}},
+                               {64, 96, 2, 0.f, false, -1, {0.723f, 1.407f}}};
 // int8 64×96: two tiles per CU at M = 1024, N = 3072 (512 tiles) instead of three 64×64 ones:
 // 9.0 vs 9.6 µs on MI355X (fewer panel re-reads through L2); 128×96, 32×96, 64×128,
 // 64×192, 32-row tiles (32×32 to 32×128) and deeper rings were slower there.
@@ -78,7 +79,10 @@ const GemmConfig kF32Cfgs[] = {{128, 128, 2, 0.90f}, {128, 64, 3, 0.95f}, {64, 6
 // 256, 3 × 3: 196 tiles of 18 k-tiles, 9.8–10.4 µs instead of 13.2–14.1 with two
 // stages and 11.0 with 32×32; eight stages 10.1–11.4, eight waves 10.7: with the
 // ring this deep a k-tile costs its own operand traffic, not its latency).
-const GemmConfig kI8Cfgs[] = {{256, 256, 1, 1.00f}, {128, 128, 2, 0.60f}, {128, 64, 3, 0.70f}, {64, 64, 4, 1.00f},
+// int8 128×128 with eight waves and four stages: 2048 × 4096 → 4096 46.1 µs
+// against 53.7 with 64×96 (128×64 and 64×128 of eight waves 47.9 and 48.8); no
+// faster than 64×96 where that is two tiles per CU (1024 × 768 → 3072 8.8 / 8.3).
+const GemmConfig kI8Cfgs[] = {{256, 256, 1, 1.00f}, {128, 128, 1, 1.10f}, {128, 64, 3, 0.70f}, {64, 64, 4, 1.00f},
                               {64, 96, 3, 1.06f}, {32, 32, 4, 0.60f, true}, {64, 64, 2, 1.20f, true}};
 
 }  // namespace

@@ -78,10 +78,10 @@ int kind_size(GemmKind k) { return k == KIND_F32 ? 4 : (k == KIND_I8 || k == KIN
 // Picks the tile configuration with the least estimated time. Kinds with
 // measured costs: rounds of num_cus·occupancy tiles, each a fixed 4 µs (launch
 // or refill, prologue, store) plus kt k-tiles at the cost of its most loaded
-// CU; a round that leaves CUs idle runs its tiles up to 30% faster when they are
-// large (64×64 and up: less traffic and power per CU; both numbers from the
-// measurements the costs come from). Other kinds: full rounds weighted by area
-// and eff. Deep-ring entries marked one_round apply only when a single round
+// CU; a round that leaves CUs idle runs the bf16 kinds' tiles up to 30% faster
+// when they are large (64×64 and up: less traffic and power per CU; both numbers
+// from the measurements the costs come from). int8: full rounds weighted by
+// area and eff. Deep-ring entries marked one_round apply only when a single round
 // holds every tile. force >= 0 (INGOT_GEMM_CFG) picks that entry when it exists.
 int pick_config(GemmKind kind, int64_t M, int64_t N, int64_t kt, int64_t batch, int num_cus, int force) {
     const GemmConfig* c;
@@ -92,19 +92,22 @@ int pick_config(GemmKind kind, int64_t M, int64_t N, int64_t kt, int64_t batch, 
     for (int i = 0; i < n; ++i) {
         const bool timed = c[i].cost[0] > 0.f;
         if (!timed && c[i].eff <= 0.f) continue;  // reached only as another entry's deep variant
-        const int64_t tiles = ((M + c[i].bm - 1) / c[i].bm) * ((N + c[i].bn - 1) / c[i].bn) * batch;
+        // M, N < 2^31: 32-bit quotients, and none where one round holds every
+        // tile (the smallest calls are bound by the host)
+        const int64_t tiles = (int64_t)(((uint32_t)M + c[i].bm - 1) / (uint32_t)c[i].bm) *
+                              (((uint32_t)N + c[i].bn - 1) / (uint32_t)c[i].bn) * batch;
         const int64_t slots = (int64_t)num_cus * c[i].occupancy;
-        const int64_t rounds = (tiles + slots - 1) / slots;
+        const int64_t rounds = tiles <= slots ? 1 : (tiles + slots - 1) / slots;
         if (c[i].one_round && rounds > 1) continue;
         double t;
         if (timed) {
             const int64_t last = tiles - (rounds - 1) * slots;  // 1..slots tiles in the last round
-            const bool large = c[i].bm * c[i].bn >= 64 * 64;
+            const bool large = kind != KIND_F32 && c[i].bm * c[i].bn >= 64 * 64;
             const double fill = large && last < num_cus ? 0.7 + 0.3 * (double)last / num_cus : 1.0;
             t = 4.0 * rounds + kt * ((rounds - 1) * (double)c[i].cost[c[i].occupancy - 1] +
-                                     c[i].cost[(last + num_cus - 1) / num_cus - 1] * fill);
+                                     c[i].cost[last <= num_cus ? 0 : (last + num_cus - 1) / num_cus - 1] * fill);
         } else {
-            const int64_t per_cu = std::min<int64_t>(c[i].occupancy, (tiles + num_cus - 1) / num_cus);
+            const int64_t per_cu = tiles <= num_cus ? 1 : std::min<int64_t>(c[i].occupancy, (tiles + num_cus - 1) / num_cus);
             t = (double)rounds * (double)per_cu * c[i].bm * c[i].bn / c[i].eff;
         }
         if (t < best_t * 0.999) {
