@@ -13,11 +13,12 @@ hipError_t launch_gemm_bf16x2(int cfg, const GemmArgs& a, int batch, hipStream_t
         case 4: return launch_one<KIND_BF16X2, 64, 128, 2, 4, 4>(a, batch, st);
         case 5: return launch_one<KIND_BF16X2, 32, 64, 2, 2, 4>(a, batch, st);
         case 6: return launch_one<KIND_BF16X2, 128, 256, 2, 4, 2>(a, batch, st);
-        case 7: return launch_one<KIND_BF16X2, 32, 32, 2, 2, 4>(a, batch, st);
+        case 7: return launch_one<KIND_BF16X2, 32, 32, 2, 2, 6>(a, batch, st);
         case 8: return launch_one<KIND_BF16X2, 64, 64, 2, 2, 4>(a, batch, st);
         // 256×192 with the weight staged through registers: every load two k-tiles ahead
         case 9: return launch_one<KIND_BF16X2, 256, 192, 4, 2, 2, 2>(a, batch, st);
         case 10: return launch_one<KIND_BF16X2, 128, 192, 2, 4, 2>(a, batch, st);
+        case 11: return launch_one<KIND_BF16X2, 16, 32, 1, 2, 5>(a, batch, st);
     }
     return hipErrorInvalidValue;
 }

@@ -42,7 +42,15 @@ const GemmConfig kBF16Cfgs[] = {{256, 256, 1, 0.f, false, -1, {1.600f}},
                                 {192, 192, 1, 0.f, false, -1, {0.911f}}};
 // hi/lo: tiles of 128 rows hold both activation planes in a stage, which costs
 // fewer operand bytes than the taller tiles' second pass over the weight (1.28
-// against 2.56 µs for 128×192 and 256×192, half the area).
+// against 2.56 µs for 128×192 and 256×192, half the area). 16×32 with five stages
+// serves up to 16 rows and long K: half the activation bytes a k-tile of 32×32,
+// and one wave's chain of fragment reads and MFMAs hidden by the fragments read
+// ahead and by up to three workgroups per CU (M = 16, weights from HBM / cached:
+// 2048 → 6144 13.6 / 10.6 → 12.5 / 9.7 µs, 5632 → 4096 27.3 / 20.0 → 23.3 / 16.9,
+// 3584 → 19712 36.6 / 30.5 → 32.9 / 26.8); 32×64 stays better where it is one
+// round of one per CU (2048 → 11264 12.5 against 13.2). 32×32 has six stages:
+// with four the loads of a k-tile come too late (M = 64, 5632 → 4096 28.9 / 21.4
+// → 27.8 / 20.6). 16×64, 16×48, 16×16 and eight stages were level or slower.
 const GemmConfig kBF16X2Cfgs[] = {{256, 256, 1, 0.f, false, -1, {3.110f}},
                                   {256, 192, 1, 0.f, false, 9, {2.560f}},
                                   {128, 128, 1, 0.f, false, -1, {0.812f}},
@@ -50,10 +58,11 @@ const GemmConfig kBF16X2Cfgs[] = {{256, 256, 1, 0.f, false, -1, {3.110f}},
                                   {64, 128, 1, 0.f, false, -1, {0.505f}},
                                   {32, 64, 2, 0.f, false, -1, {0.229f, 0.423f}},
                                   {128, 256, 1, 0.f, false, -1, {1.551f}},
-                                  {32, 32, 3, 0.f, false, -1, {0.190f, 0.301f, 0.449f}},
+                                  {32, 32, 2, 0.f, false, -1, {0.175f, 0.320f}},
                                   {64, 64, 1, 0.f, false, -1, {0.373f}},
                                   {256, 192, 1, 0.f, false},
-                                  {128, 192, 1, 0.f, false, -1, {1.280f}}};
+                                  {128, 192, 1, 0.f, false, -1, {1.280f}},
+                                  {16, 32, 3, 0.f, false, -1, {0.150f, 0.280f, 0.410f}}};
 // f32: a k-tile is bound by its MFMAs (a tile's area per µs of cost is 7.1–9.0
 // thousand outputs, 9.0 being 147 of the 157 TFLOP/s peak), so the tiles differ
 // little but for how they divide a product over 256 CUs; 32×32 serves products

@@ -207,7 +207,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
     constexpr int IA = BM / (8 * NW), IB = BN / (8 * NW);  // 8-row DMA loads per wave per k-tile (A plane, B)
     static_assert(IA * 8 * NW == BM && IB * 8 * NW == BN, "DMA rows must split evenly over the waves");
     constexpr int STAGE = (AP * BM + BN) * KTILE_BYTES;
-    static_assert(BM % 32 == 0 && BN % 32 == 0, "tile must be a multiple of 32");
+    static_assert(WM % 16 == 0 && WN % 16 == 0, "wave tiles are whole 16 x 16 blocks");
     typedef typename AccOf<KD>::type Acc;
 
     // NS LDS stages (a ring of k-tiles). Rows are 128 bytes, unpadded; the
@@ -440,6 +440,15 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
     // half multiplies the hi plane's two half k-tiles, the second the lo plane's
     constexpr int NMF0 = (KD == KIND_F32 ? 4 : 1) * AP * TM * TN;
     constexpr int NMF1 = NMF0;
+    // AHEAD (hi/lo tiles of few blocks per wave): what bounds their k-tile is a
+    // chain, not a rate: LDS latency of the second half's fragments, MFMAs on
+    // one or few accumulators, barrier, LDS latency of the next first half. So
+    // k-tile kt+1's fragments are read whole while kt's are multiplied (two full
+    // register sets; the sums keep their order). On MI355X, cached operands:
+    // 16×32 tile at M = 16, 5632 → 4096 19.1 → 16.9 µs; 64×128 at M = 17, 2048 →
+    // 6144 19.2 → 16.7; 64×128 at M = 64, 5632 → 4096 44.4 → 38.6. Wave tiles of
+    // more blocks cover the latency with their MFMAs and would need the registers.
+    constexpr bool AHEAD = KD == KIND_BF16X2 && AP == 2 && TM * TN <= 4;
     FragA fa0, fa1;
     FragB fb0, fb1;
     // The epilogue terms: raw loads issued right after k-tile 0's DMA, the
@@ -554,7 +563,36 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
         if (kt < KT) rs_step(kt, std::integral_constant<int, 0>(), rb1);
     }
     int st = 0;  // ring slot of k-tile kt
-    for (int kt = 0; kt < (RS ? 0 : KT); ++kt) {
+    // AHEAD: kt's fragments of both halves were read during kt − 1.
+    auto ahead_step = [&](int kt, const FragA& c0, const FragB& d0, const FragA& c1, const FragB& d1, FragA& n0, FragB& e0,
+                          FragA& n1, FragB& e1) {
+        char* cur = lds + st * SSTRIDE;
+        st = st + 1 == NS ? 0 : st + 1;
+        wait_dma_groups<G, NS>(NS - 2);
+        kloop_barrier();  // cur fully read by every wave; k-tile kt+1 landed
+        __builtin_amdgcn_sched_barrier(0);
+        read_frags(lds + st * SSTRIDE, 0, n0, e0);  // after the last k-tile: unused
+        read_frags(lds + st * SSTRIDE, 1, n1, e1);
+        dma(cur, kt + NS);
+#pragma unroll
+        for (int pl = 0; pl < AP; ++pl) {
+            mma_plane(c0[pl], d0);
+            mma_plane(c1[pl], d1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (AHEAD) {
+        FragA ga0, ga1;
+        FragB gb0, gb1;
+        read_frags(lds, 1, fa1, fb1);
+        int kt = 0;
+        for (; kt + 1 < KT; kt += 2) {
+            ahead_step(kt, fa0, fb0, fa1, fb1, ga0, gb0, ga1, gb1);
+            ahead_step(kt + 1, ga0, gb0, ga1, gb1, fa0, fb0, fa1, fb1);
+        }
+        if (kt < KT) ahead_step(kt, fa0, fb0, fa1, fb1, ga0, gb0, ga1, gb1);
+    }
+    for (int kt = 0; kt < (RS || AHEAD ? 0 : KT); ++kt) {
         char* cur = lds + st * SSTRIDE;
         const int st1 = st + 1 == NS ? 0 : st + 1;
         read_frags(cur, 1, fa1, fb1);

@@ -447,7 +447,7 @@ def test_gemv_epilogue(sess, m):
 # ragged edges in M, N and K, with a bias and an activation in the epilogue
 # (int8: the column-sum correction and fused dequantisation). Indices follow the
 # configuration tables of gemm_mfma.hip.
-GEMM_CFGS = {"f32": range(7), "bf16": range(12), "bf16x2": range(11), "i8": range(7)}
+GEMM_CFGS = {"f32": range(7), "bf16": range(12), "bf16x2": range(12), "i8": range(7)}
 
 
 @pytest.mark.parametrize("kind,cfg", [(k, c) for k, r in GEMM_CFGS.items() for c in r])
@@ -486,6 +486,28 @@ def test_gemm_forced_tile_configs(env_session, kind, cfg, m, n, k):
                        act_code=L.ACT_GELU_ERF, **({"b_dtype": bdt} if bdt is not None else {}))
     assert_close(y.numpy(), want, nstar_tol(k, a, wide), f"{kind} cfg {cfg}")
     w.free()
+
+
+# The hi/lo tiles that read a k-tile's fragments one k-tile ahead, against the 128 x 128 tile, which does not (the same
+# sums in the same order: equal bits): one k-tile, an odd and an even number of them, fewer and more than the ring
+# holds; M at the edges of the 16-row tile; N ragged.
+@pytest.mark.parametrize("cfg", [4, 5, 7, 8, 11])
+def test_gemm_split_ahead_tiles_equal_bits(env_session, cfg):
+    rng = np.random.default_rng(cfg)
+    ref, sess = env_session(INGOT_GEMM_CFG=2), env_session(INGOT_GEMM_CFG=cfg)
+    for m, n, k in [(17, 40, 64), (33, 33, 65), (18, 130, 192), (31, 97, 256), (17, 70, 400), (64, 65, 1030)]:
+        announce(f"gemm ahead cfg={cfg} m={m} n={n} k={k}")
+        a, bt = rng.normal(0, 1, (m, k)).astype(np.float32), bf16_weights(rng, (n, k))
+        out = []
+        for s in (ref, sess):
+            w = s.upload_weight(bt, trans=True, pack_dtype=L.DT_BF16, src_dtype=L.DT_BF16)
+            y = s.empty(L.DT_F32, (m, n))
+            s.gemm(s.to_device(a), w, y, m)
+            out.append(y.numpy())
+            w.free()
+        assert np.array_equal(out[0], out[1]), f"cfg {cfg} m {m} n {n} k {k}"
+        want = oracle.gemm(a, bt, trans_b=True, b_dtype=oracle.BF16)
+        assert_close(out[1], want, nstar_tol(k, a, oracle.bf16_to_f32(bt)), f"ahead cfg {cfg}")
 
 
 @pytest.mark.parametrize("cfg", ["10", "11", "12", "13", "14", "15", "16", "17", "18", "19", "20", "21", "22",
