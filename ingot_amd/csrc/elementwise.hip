@@ -2,6 +2,7 @@
 // the standalone activation / bias pass, the f32 → bf16 cast and fills.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "kernels.hpp"
 
@@ -280,142 +281,158 @@ __global__ __launch_bounds__(256) void pack_a_flat_kernel(const float* __restric
 }
 
 // ---- elementwise passes ----
-// A pass sees its tensor as rows × cols (the last row may be short: n counts
-// the elements) with per-column or per-row operands, so that no element is
-// divided for its index: 2^txs threads side by side on a row, V neighbouring
-// elements each, loaded and stored together at any element alignment. HBM-bound:
-// one element a thread with a 64-bit division and remainder for a per-axis
-// scale, DequantizeLinear of 4000 × 4000 int8 per row took 53 µs on MI355X and
-// the GELU of its result 31 µs; these take 27 and 21 µs. V is 4 where that
-// fills the chip; small tensors take one element a thread, which is done
-// sooner (400 × 100 int32 per column 2.6 µs, 2.9 with four).
-struct Grid2 {
-    int64_t n, rows, cols;
-    int v, txs;
-    Grid2(int64_t n_, int64_t cols_) : n(n_), rows((n_ + cols_ - 1) / cols_), cols(cols_), v(n_ >> 19 ? 4 : 1), txs(0) {
-        while (txs < 8 && ((int64_t)v << txs) < cols) ++txs;
+// A thread takes V neighbouring elements of the flat tensor, loaded and stored
+// together at any element alignment. HBM-bound when large, by launch and load
+// latency when small. A per-axis operand (scale, zero point, bias) costs two
+// multiplications by a reciprocal per V elements, and its loads wait for nothing
+// but the index, like the element's own. V is 4 where that fills the chip,
+// else 1, which is done sooner (400 × 100 int32 per column 2.5 µs on MI355X, 2.9
+// with four). DequantizeLinear and the GELU of its result, kernel times on
+// MI355X: 4000 × 4000 int8 per row 15.0 and 19.7 µs (one element a thread with
+// a 64-bit division each 38.6 and 30.9; a grid over rows and columns 17.9 and
+// 20.6), 1024 × 3072 int32 per column 8.0 and 6.4 (9.5 and 8.1; 8.5 and 7.1),
+// 100000 × 7 int32 per row 3.0 and 3.0 (3.8 and 3.4; 4.8 and 3.7), 4096 × 65 per
+// column 2.7 and 2.6 (2.9 and 2.6; 3.2 and 3.0).
+
+// Which of `count` operands element i takes: (i / inner) % count. Below 2^31
+// elements both quotients are exact as the upper half of a product with
+// ceil(2^(31 + l) / d), l = ceil(log2 d), shifted by l − 1 (Granlund and
+// Montgomery); WIDE divides in 64 bits.
+struct Axis {
+    int64_t inner, count;
+    uint32_t mi, mc;  // 0: a divisor of 1
+    int si, sc;
+    Axis(int64_t n, int64_t inner_, int64_t count_)
+        : inner(std::min(std::max<int64_t>(inner_, 1), n)), count(std::min(count_, n)) {
+        reciprocal(inner, &mi, &si);
+        reciprocal(count, &mc, &sc);
     }
-    dim3 grid() const {
-        const int64_t per = 256 >> txs;
-        return dim3((unsigned)((((cols + v - 1) / v) + (1 << txs) - 1) >> txs),
-                    (unsigned)std::min<int64_t>((rows + per - 1) / per, 65535));
+    static void reciprocal(int64_t d, uint32_t* m, int* s) {
+        int l = 0;
+        while (l < 31 && ((int64_t)1 << l) < d) ++l;
+        *m = l ? (uint32_t)((((uint64_t)1 << (31 + l)) + d - 1) / d) : 0u;
+        *s = l ? l - 1 : 0;
     }
 };
 
-// This thread's first column; body(row, index of its first element, how many of the V are there) for its rows.
-template <int V>
-__device__ __forceinline__ int64_t first_col(int txs) {
-    return (((int64_t)blockIdx.x << txs) + (threadIdx.x & ((1 << txs) - 1))) * V;
-}
+// The operand index of element i and of the elements after it.
+template <bool WIDE>
+struct AxisAt {
+    typedef std::conditional_t<WIDE, int64_t, uint32_t> I;
+    I c, r;
+    __device__ __forceinline__ AxisAt(const Axis& a, int64_t i) {
+        if constexpr (WIDE) {
+            const int64_t q = i / a.inner;
+            r = i - q * a.inner, c = q % a.count;
+        } else {
+            const uint32_t u = (uint32_t)i;
+            const uint32_t q = a.mi ? __umulhi(u, a.mi) >> a.si : u;
+            r = u - q * (uint32_t)a.inner;
+            c = q - (a.mc ? __umulhi(q, a.mc) >> a.sc : q) * (uint32_t)a.count;
+        }
+    }
+    __device__ __forceinline__ void next(const Axis& a) {
+        if (++r == (I)a.inner) {
+            r = 0;
+            if (++c == (I)a.count) c = 0;
+        }
+    }
+};
+
+struct Grid1 {
+    int v;
+    unsigned blocks;
+    explicit Grid1(int64_t n) : v(n >> 19 ? 4 : 1), blocks(grid_for(n, 256 * v)) {}
+};
+
+// body(width, index of the first element): this thread's chunks of V, and the elements of a short last one singly (a
+// chunk that may be short would be loaded in pieces).
 template <int V, typename Body>
-__device__ __forceinline__ void walk_rows(int64_t n, int64_t rows, int64_t cols, int txs, int64_t col, Body body) {
-    const int64_t step = (int64_t)gridDim.y * (256 >> txs);
-    for (int64_t r = (int64_t)blockIdx.y * (256 >> txs) + (threadIdx.x >> txs); r < rows; r += step) {
-        const int64_t i = r * cols + col;
-        if (i < n) body(r, i, (int)min(min(cols - col, n - i), (int64_t)V));
-    }
-}
-
-template <int V, typename T>
-__device__ __forceinline__ void load_v(T (&v)[V], const T* p, int have) {
-    if (have == V) {
-        __builtin_memcpy(v, p, V * sizeof(T));
-    } else {
-#pragma unroll
-        for (int e = 0; e < V; ++e)  // static indexes: v stays in registers
-            if (e < have) v[e] = p[e];
-    }
-}
-template <int V, typename T>
-__device__ __forceinline__ void store_v(T* p, const T (&v)[V], int have) {
-    if (have == V) {
-        __builtin_memcpy(p, v, V * sizeof(T));
-    } else {
-#pragma unroll
-        for (int e = 0; e < V; ++e)
-            if (e < have) p[e] = v[e];
-    }
-}
-
-__device__ __forceinline__ int32_t load_zp(const void* p, int dt, int64_t i) {
-    switch (dt) {
-        case INGOT_DT_U8: return (int32_t)((const uint8_t*)p)[i];
-        case INGOT_DT_I8: return (int32_t)((const int8_t*)p)[i];
-        default: return ((const int32_t*)p)[i];
-    }
-}
-
-// COL: one scale (and zero point) per column; else one per row, row r taking r % n_scale.
-template <typename T, bool COL, int V>
-__global__ __launch_bounds__(256) void dequant_kernel(const T* x, int64_t n, int64_t rows, int64_t cols, int txs,
-                                                      const float* scale, int64_t n_scale, const void* zp, int zp_dt,
-                                                      int64_t n_zp, float* y) {
-    const int64_t col = first_col<V>(txs);
-    if (col >= cols) return;
-    float sc[V];
-    int32_t z[V];
-    if constexpr (COL) {
-#pragma unroll
-        for (int e = 0; e < V; ++e) {
-            const int64_t c = min(col + e, cols - 1);
-            sc[e] = scale[c];
-            z[e] = zp ? load_zp(zp, zp_dt, n_zp > 1 ? c : 0) : 0;
+__device__ __forceinline__ void walk(int64_t n, Body body) {
+    const int64_t step = (int64_t)gridDim.x * 256 * V;
+    for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V; i < n; i += step) {
+        if (V == 1 || i + V <= n) {
+            body(std::integral_constant<int, V>(), i);
+        } else {
+            for (; i < n; ++i) body(std::integral_constant<int, 1>(), i);
         }
     }
-    walk_rows<V>(n, rows, cols, txs, col, [&](int64_t r, int64_t i, int have) {
-        T v[V];
-        load_v<V>(v, x + i, have);
-        float rs = 0.f;
-        int32_t rz = 0;
-        if constexpr (!COL) {
-            const int64_t c = n_scale == 1 ? 0 : rows >> 32 ? r % n_scale : (int64_t)((uint32_t)r % (uint32_t)n_scale);
-            rs = scale[c];
-            rz = zp ? load_zp(zp, zp_dt, n_zp > 1 ? c : 0) : 0;
-        }
-        float f[V];
+}
+
+// z[e] = zero point c[e].
+template <int W, typename Z, typename I>
+__device__ __forceinline__ void load_zp(int32_t (&z)[W], const void* zp, const I (&c)[W]) {
 #pragma unroll
-        for (int e = 0; e < V; ++e) f[e] = (float)wrap_add((int32_t)v[e], -(COL ? z[e] : rz)) * (COL ? sc[e] : rs);
-        store_v<V>(y + i, f, have);
+    for (int e = 0; e < W; ++e) z[e] = (int32_t)((const Z*)zp)[c[e]];
+}
+
+// AXIS 0: one scale for all; 1: per axis; 2: per axis, 2^31 elements or more.
+template <typename T, int AXIS, int V>
+__global__ __launch_bounds__(256) void dequant_kernel(const T* x, int64_t n, const float* scale, Axis axis,
+                                                      const void* zp, int zp_dt, int zp_each, float* y) {
+    walk<V>(n, [&](auto width, int64_t i) {
+        constexpr int W = decltype(width)::value;
+        T v[W];
+        __builtin_memcpy(v, x + i, sizeof v);
+        // operand indexes of the elements
+        std::conditional_t<AXIS == 2, int64_t, uint32_t> c[W] = {};
+        if constexpr (AXIS != 0) {
+            AxisAt<AXIS == 2> at(axis, i);
+#pragma unroll
+            for (int e = 0; e < W; ++e) c[e] = at.c, at.next(axis);
+        }
+        float sc[W];
+#pragma unroll
+        for (int e = 0; e < W; ++e) sc[e] = scale[c[e]];
+        int32_t z[W] = {};
+        if (zp) {
+            if (AXIS != 0 && !zp_each) {
+#pragma unroll
+                for (int e = 0; e < W; ++e) c[e] = 0;
+            }
+            if (zp_dt == INGOT_DT_U8) load_zp<W, uint8_t>(z, zp, c);
+            else if (zp_dt == INGOT_DT_I8) load_zp<W, int8_t>(z, zp, c);
+            else load_zp<W, int32_t>(z, zp, c);
+        }
+        float f[W];
+#pragma unroll
+        for (int e = 0; e < W; ++e) f[e] = (float)wrap_add((int32_t)v[e], -z[e]) * sc[e];
+        __builtin_memcpy(y + i, f, sizeof f);
     });
 }
 
-// y = post(act(x + bias[column])), bias optional.
-template <int ACT, int V>
-__global__ __launch_bounds__(256) void activation_kernel(const float* x, float* y, int64_t n, int64_t rows, int64_t cols,
-                                                         int txs, const float* bias, float a, float b, int post, float ps,
-                                                         float pb) {
-    const int64_t col = first_col<V>(txs);
-    if (col >= cols) return;
-    float bi[V];
-    if (bias) {
+// y = post(act(x + bias[column])), bias optional (WIDE: 2^31 elements or more).
+template <int ACT, bool WIDE, int V>
+__global__ __launch_bounds__(256) void activation_kernel(const float* x, float* y, int64_t n, const float* bias, Axis axis,
+                                                         float a, float b, int post, float ps, float pb) {
+    walk<V>(n, [&](auto width, int64_t i) {
+        constexpr int W = decltype(width)::value;
+        float v[W];
+        __builtin_memcpy(v, x + i, sizeof v);
+        if (bias) {
+            AxisAt<WIDE> at(axis, i);
 #pragma unroll
-        for (int e = 0; e < V; ++e) bi[e] = bias[min(col + e, cols - 1)];
-    }
-    walk_rows<V>(n, rows, cols, txs, col, [&](int64_t, int64_t i, int have) {
-        float v[V];
-        load_v<V>(v, x + i, have);
+            for (int e = 0; e < W; ++e) v[e] += bias[at.c], at.next(axis);
+        }
 #pragma unroll
-        for (int e = 0; e < V; ++e) {
-            if (bias) v[e] += bi[e];
+        for (int e = 0; e < W; ++e) {
             if (ACT != INGOT_ACT_NONE) v[e] = apply_act(v[e], ACT, a, b);
             if (post) v[e] = v[e] * ps + pb;
         }
-        store_v<V>(y + i, v, have);
+        __builtin_memcpy(y + i, v, sizeof v);
     });
 }
 
 template <int V>
-__global__ __launch_bounds__(256) void cast_bf16_kernel(const float* x, uint16_t* y, int64_t n, int64_t rows,
-                                                        int64_t cols, int txs) {
-    const int64_t col = first_col<V>(txs);
-    if (col >= cols) return;
-    walk_rows<V>(n, rows, cols, txs, col, [&](int64_t, int64_t i, int have) {
-        float v[V];
-        load_v<V>(v, x + i, have);
-        uint16_t h[V];
+__global__ __launch_bounds__(256) void cast_bf16_kernel(const float* x, uint16_t* y, int64_t n) {
+    walk<V>(n, [&](auto width, int64_t i) {
+        constexpr int W = decltype(width)::value;
+        float v[W];
+        __builtin_memcpy(v, x + i, sizeof v);
+        uint16_t h[W];
 #pragma unroll
-        for (int e = 0; e < V; ++e) h[e] = f32_to_bf16(v[e]);
-        store_v<V>(y + i, h, have);
+        for (int e = 0; e < W; ++e) h[e] = f32_to_bf16(v[e]);
+        __builtin_memcpy(y + i, h, sizeof h);
     });
 }
 
@@ -470,21 +487,19 @@ hipError_t launch_pack_a(const void* src, int src_dtype, int64_t lda, int trans,
 
 hipError_t launch_dequant(const void* x, int x_dtype, int64_t n, const float* scale, int64_t n_scale, int64_t inner,
                           const void* zp, int zp_dtype, int64_t n_zp, float* y, hipStream_t st) {
-    if (inner < 1) inner = 1;
-    // element i takes scale (i / inner) % n_scale: per column when inner is 1,
-    // per row of `inner` else; one scale for all: any row length
-    const bool col = n_scale > 1 && inner == 1;
-    const Grid2 g(n, n_scale == 1 ? std::min<int64_t>(n, 1024) : (col ? n_scale : inner));
+    if (n <= 0) return hipSuccess;
+    const Grid1 g(n);
+    const Axis axis(n, inner, n_scale);
     const auto launch = [&](auto kernel, auto t) {
-        typedef decltype(t) T;
-        hipLaunchKernelGGL(kernel, g.grid(), dim3(256), 0, st, (const T*)x, n, g.rows, g.cols, g.txs, scale, n_scale, zp,
-                           zp_dtype, n_zp, y);
+        hipLaunchKernelGGL(kernel, dim3(g.blocks), dim3(256), 0, st, (const decltype(t)*)x, n, scale, axis, zp, zp_dtype,
+                           n_zp > 1 ? 1 : 0, y);
         return hipGetLastError();
     };
     const auto go = [&](auto t) {
         typedef decltype(t) T;
-        if (g.v == 1) return col ? launch(dequant_kernel<T, true, 1>, t) : launch(dequant_kernel<T, false, 1>, t);
-        return col ? launch(dequant_kernel<T, true, 4>, t) : launch(dequant_kernel<T, false, 4>, t);
+        if (n_scale == 1) return g.v == 1 ? launch(dequant_kernel<T, 0, 1>, t) : launch(dequant_kernel<T, 0, 4>, t);
+        if (n >> 31) return launch(dequant_kernel<T, 2, 4>, t);
+        return g.v == 1 ? launch(dequant_kernel<T, 1, 1>, t) : launch(dequant_kernel<T, 1, 4>, t);
     };
     switch (x_dtype) {
         case INGOT_DT_U8: return go((uint8_t)0);
@@ -497,14 +512,19 @@ hipError_t launch_dequant(const void* x, int x_dtype, int64_t n, const float* sc
 hipError_t launch_activation(const float* x, float* y, int64_t rows, int64_t cols, const float* bias, int act, float a,
                              float b, int post, float ps, float pb, hipStream_t st) {
     const int64_t n = rows * cols;
-    const Grid2 g(n, bias ? cols : std::min<int64_t>(n, 1024));
+    if (n <= 0) return hipSuccess;
+    const Grid1 g(n);
+    const Axis axis(n, 1, cols);
     const auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, g.grid(), dim3(256), 0, st, x, y, n, g.rows, g.cols, g.txs, bias, a, b, post, ps, pb);
+        hipLaunchKernelGGL(kernel, dim3(g.blocks), dim3(256), 0, st, x, y, n, bias, axis, a, b, post, ps, pb);
         return hipGetLastError();
     };
     switch (act) {
-#define INGOT_ACT_CASE(A) \
-    case A: return g.v == 1 ? launch(activation_kernel<A, 1>) : launch(activation_kernel<A, 4>);
+#define INGOT_ACT_CASE(A)                                      \
+    case A:                                                    \
+        return g.v == 1  ? launch(activation_kernel<A, false, 1>) \
+               : n >> 31 ? launch(activation_kernel<A, true, 4>)  \
+                         : launch(activation_kernel<A, false, 4>);
         INGOT_ACT_CASE(INGOT_ACT_NONE)
         INGOT_ACT_CASE(INGOT_ACT_RELU)
         INGOT_ACT_CASE(INGOT_ACT_GELU_ERF)
@@ -521,11 +541,12 @@ hipError_t launch_activation(const float* x, float* y, int64_t rows, int64_t col
 }
 
 hipError_t launch_cast_bf16(const float* x, uint16_t* y, int64_t n, hipStream_t st) {
-    const Grid2 g(n, std::min<int64_t>(n, 1024));
+    if (n <= 0) return hipSuccess;
+    const Grid1 g(n);
     if (g.v == 1)
-        hipLaunchKernelGGL(cast_bf16_kernel<1>, g.grid(), dim3(256), 0, st, x, y, n, g.rows, g.cols, g.txs);
+        hipLaunchKernelGGL(cast_bf16_kernel<1>, dim3(g.blocks), dim3(256), 0, st, x, y, n);
     else
-        hipLaunchKernelGGL(cast_bf16_kernel<4>, g.grid(), dim3(256), 0, st, x, y, n, g.rows, g.cols, g.txs);
+        hipLaunchKernelGGL(cast_bf16_kernel<4>, dim3(g.blocks), dim3(256), 0, st, x, y, n);
     return hipGetLastError();
 }
 

@@ -299,6 +299,54 @@ def test_dequantize_views(sess, n, n_scale, inner, dtype):
         np.testing.assert_array_equal(y.numpy(), oracle.dequantize_linear(x, sc, inner=inner, zp=zp))
 
 
+@pytest.mark.parametrize("n,n_scale,inner", [(6, 2, 1 << 42), (5, 9, 1), (7, 3, 7), (700003, 5, 7), (1 << 19, 3, 1),
+                                             (530001, 65, 1), (600007, 2, 300000), (524289, 1 << 19, 1),
+                                             (530000, 1, 3), (786433, 255, 257)])
+def test_dequantize_axes(sess, n, n_scale, inner):
+    """Axes longer than the tensor, of one and of odd lengths, at sizes that take four elements a thread, with a short
+    last chunk: exactly the oracle's values."""
+    announce(f"dequant axes n={n} scales={n_scale} inner={inner}")
+    rng = np.random.default_rng(n + n_scale)
+    x = rng.integers(-128, 128, n).astype(np.int8)
+    sc = rng.uniform(0.01, 0.1, n_scale).astype(np.float32)
+    for zp in (None, rng.integers(-100, 100, n_scale).astype(np.int8)):
+        y = sess.empty(L.DT_F32, (n,))
+        sess.dequantize_linear(dev(sess, x, L.DT_I8), dev(sess, sc), y, inner=inner,
+                               zp=None if zp is None else dev(sess, zp, L.DT_I8))
+        np.testing.assert_array_equal(y.numpy(), oracle.dequantize_linear(x, sc, inner=min(inner, n), zp=zp))
+
+
+def test_dequantize_wide(sess):
+    """2^31 elements and more (64-bit indexes): the first, the middle and the last ones."""
+    announce("dequant of 2^31 + 11 elements")
+    n, sc = (1 << 31) + 11, np.array([0.5, 0.25, 2.0], np.float32)
+    x, y = sess.empty(L.DT_U8, (n,)), sess.empty(L.DT_F32, (n,))
+    sess.memset(x, 7)
+    sess.dequantize_linear(x, dev(sess, sc), y, inner=5)
+    for first in (0, (1 << 30) + 3, n - 64):
+        got = np.empty(64, np.float32)
+        L.check(sess.lib.ingot_rocm_memcpy_d2h(sess.h, got.ctypes.data, y.ptr + 4 * first, got.nbytes))
+        want = np.float32(7) * sc[(np.arange(first, first + 64) // 5) % 3]
+        np.testing.assert_array_equal(got, want)
+    x.free()
+    y.free()
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (1, 1027), (5, 3), (9, 257), (33, 1028), (1100, 513), (3, 200001)])
+def test_activation_bias_axes(sess, rows, cols):
+    """The bias row at sizes that take one and four elements a thread (x + bias is one rounded sum; ReLU is exact),
+    in place too."""
+    announce(f"activation bias axes {rows}x{cols}")
+    rng = np.random.default_rng(rows + cols)
+    x = rng.normal(0, 1, (rows, cols)).astype(np.float32)
+    b = rng.normal(0, 1, cols).astype(np.float32)
+    dx, y = dev(sess, x), sess.empty(L.DT_F32, (rows, cols))
+    sess.activation(dx, y, rows, cols, L.ACT_RELU, bias=dev(sess, b))
+    np.testing.assert_array_equal(y.numpy(), np.maximum(x + b, 0))
+    sess.activation(dx, dx, rows, cols, L.ACT_RELU, bias=dev(sess, b))
+    np.testing.assert_array_equal(dx.numpy(), np.maximum(x + b, 0))
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 1), (1, 1027), (5, 3), (9, 257), (33, 1028)])
 def test_activation_bias_views(sess, rows, cols):
     """The bias row at widths around 4 elements and a thread row (x + bias is one rounded sum; ReLU is exact), the

@@ -8,6 +8,7 @@ Each model follows the index arithmetic of one kernel and checks a property that
 - gemv_bf16.hip reduce_store: the reduce-scatter butterfly gives every sum bit-identical to a full butterfly,
   and exactly one store lane holds each sum;
 - gemv_bf16.hip gemv_dma_kernel: the staged x blocks meet the weight bytes of the same k in the FMAs.
+- elementwise.hip Axis: the quotients by reciprocal multiplication are exact below 2^31.
 """
 import numpy as np
 import pytest
@@ -133,3 +134,19 @@ def test_dma_gemv_x_blocks_meet_weight_k(mm, chunks, k):
                 for e in range(8):
                     acc[row, :, lane] += blocks[:, c, e >> 2, lane, e & 3] * wl[e]
     assert np.array_equal(acc.sum(axis=2), w @ x.T)
+
+
+# elementwise.hip Axis: quotients as the upper half of a 32 x 32-bit product.
+@pytest.mark.parametrize("d", [1, 2, 3, 5, 7, 64, 65, 255, 256, 257, 1000003, (1 << 20) - 1, (1 << 30) - 1, 1 << 30,
+                               (1 << 30) + 1, (1 << 31) - 1])
+def test_axis_reciprocal_quotients(d):
+    """i / d for every i below 2^31 from ceil(2^(31 + l) / d): at 0, around multiples of d and at the end of the range."""
+    lg = (d - 1).bit_length()
+    m = ((1 << (31 + lg)) + d - 1) // d if lg else 0
+    assert m < 1 << 32
+    top = (1 << 31) - 1
+    rng = np.random.default_rng(d)
+    for q in {0, 1, 2, top // d} | {int(v) for v in rng.integers(0, top // d + 1, 500)}:
+        for i in (q * d - 1, q * d, q * d + 1, q * d + d - 1, top):
+            if 0 <= i <= top:
+                assert (((i * m) >> 32) >> (lg - 1) if lg else i) == i // d
