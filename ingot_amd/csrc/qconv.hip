@@ -22,7 +22,7 @@
 //    inside the image (padded taps contribute exactly 0). Used for narrow
 //    groups, where a GEMM would be a sliver, and for depthwise forms the strip
 //    kernel does not hold (kernel rows over 8 taps, dilated rows, strips over
-//    its LDS).
+//    its LDS) or that give its waves too little work (launch_qconv_depthwise).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -529,7 +529,7 @@ constexpr int DW_LDS = 64 * 1024;
 
 hipError_t launch_qconv_depthwise(const void* x, int x_u8, const QconvGeom& g, const int8_t* w, int64_t ldw,
                                   const int32_t* bias, const float* mult, int32_t zx, float zy, int y_u8, void* y,
-                                  hipStream_t st, bool* done) {
+                                  hipStream_t st, bool any, bool* done) {
     *done = false;
     // what the kernel's windows and 16-bit index arithmetic hold; anything else is the direct kernel's
     if (g.Cg != 1 || g.KW > 8 || g.dw != 1 || g.KH > 64 || g.W >= (1 << 15) || g.OW >= (1 << 15) || g.pl >= (1 << 12) ||
@@ -570,8 +570,10 @@ hipError_t launch_qconv_depthwise(const void* x, int x_u8, const QconvGeom& g, c
     // whole 8-byte row pieces, indexes the magic division holds
     p.ipp = (uint32_t)p.qpr * (uint32_t)((g.OH + 3) / 4);
     const int64_t blocks4 = (int64_t)p.planes * p.ipp;
+    // (one output row at stride 2 leaves three quarters of a lane's rows unused: 32768 planes of 2 × 8, 3 × 3 4.7 µs,
+    // 4.2 in the direct kernel)
     if (g.KH == g.KW && (g.KH == 3 || g.KH == 5) && g.sh == g.sw && g.sw <= 2 && g.dh == 1 && g.W >= 8 &&
-        (int64_t)p.qpr * ((g.OH + 3) / 4) + 256 < (1 << 16) && blocks4 < (1ll << 31)) {
+        (any || g.sw == 1 || g.OH > 1) && (int64_t)p.qpr * ((g.OH + 3) / 4) + 256 < (1 << 16) && blocks4 < (1ll << 31)) {
         p.ipp_magic = magic((int)p.ipp);
         const dim3 bg((unsigned)((blocks4 + 255) / 256));
         if (g.KH == 3 && g.sw == 1) hipLaunchKernelGGL((qconv_dw_block_kernel<1, 3>), bg, dim3(256), 0, st, p);
@@ -581,6 +583,20 @@ hipError_t launch_qconv_depthwise(const void* x, int x_u8, const QconvGeom& g, c
         *done = true;
         return hipGetLastError();
     }
+    // A strip costs a wave about 0.8 ns of the chip and 5–6 µs from launch to
+    // store however little it holds; the direct kernel about 6 ps + 0.44 ps a tap
+    // and output, and 3 µs + 0.12 a tap. So the strip kernel takes what holds
+    // enough products per strip and per call, and a stride only with the taps
+    // that pay for the input it skips (MI355X, strip / direct µs: 30720 planes of
+    // 7 × 7, 3 × 3 25.4 / 16.0, 5 × 5 30.5 / 25.1, 24576 of 7 × 7, 7 × 7 26.6 / 32.5;
+    // 32768 of 1 × 1 26.3 / 3.5; 32 of 28 × 28, 1 × 1 6.5 / 3.1, 768 of 56 × 56 8.0 /
+    // 14.0; 2 × 2 stride 2, 56 × 56 10.7 / 7.0, 4 × 4 10.8 / 11.4; 512 of 112 × 112
+    // stride 3, 3 × 3 11.9 / 10.3, 7 × 7 16.5 / 31.0).
+    const int64_t taps = (int64_t)g.KH * g.KW, outs = (int64_t)p.th * g.OW;
+    if (!any && (outs * (13 + taps) < 2000 ||
+                 (int64_t)p.planes * g.OH * g.OW * (13 + taps) + 284000 * taps < 6800000 ||
+                 taps < 16 * (int64_t)(std::max(g.sh, g.sw) - 1)))
+        return hipSuccess;
 #define INGOT_DW(SW, NWD) hipLaunchKernelGGL((qconv_dw_kernel<SW, NWD>), grid, dim3(256), lds, st, p)
     if (nwd == 1) {
         if (g.sw == 1) INGOT_DW(1, 1);

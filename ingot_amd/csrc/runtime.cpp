@@ -960,16 +960,17 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
     // one launch beats the layout and the GEMM (on MI355X, kernels alone, direct /
     // GEMM: 4 × 128 × 28 × 28 outputs of K = 3 5.7 / 7.4 µs, of K = 19 12.4 / 8.0;
     // 8 × 32 × 32 × 32 of K = 27 9.2 / 8.1: the line is 2^22 products).
-    // INGOT_QCONV_PATH=1/2/3 forces direct / pixel GEMM / im2col GEMM (tests run
-    // the routes on the same cases).
+    // INGOT_QCONV_PATH=1/2/3/4 forces direct / pixel GEMM / im2col GEMM / the
+    // depthwise kernels wherever they hold the form (tests run the routes on the
+    // same cases).
     const int path = s->qconv_path;
     const int64_t kgl = round_up(K, 128);
-    const bool gemm = path >= 2 || (path != 1 && Mg >= 16 && (K >= 32 || total * K >= (1ll << 22)));
+    const bool gemm = path == 2 || path == 3 || (path == 0 && Mg >= 16 && (K >= 32 || total * K >= (1ll << 22)));
     if (!gemm) {
         if (path != 1) {
             bool done = false;
             hipError_t e = launch_qconv_depthwise(a->d_x, u8 ? 1 : 0, g, (const int8_t*)w->data, w->ldk, a->d_bias,
-                                                  a->d_mult, a->zx, (float)a->zy, yu8, a->d_y, s->stream, &done);
+                                                  a->d_mult, a->zx, (float)a->zy, yu8, a->d_y, s->stream, path == 4, &done);
             if (e != hipSuccess) return hip_fail(e, "qconv depthwise");
             if (done) return INGOT_OK;
         }

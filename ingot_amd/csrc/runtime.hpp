@@ -32,7 +32,7 @@ struct ingot_rocm_session {
     // configuration, INGOT_GEMV_CFG a GEMV launch configuration,
     // INGOT_I8G_ROWS the int8 GEMV rows per wave, INGOT_NO_GEMV sends decode
     // rows to the GEMM, INGOT_QCONV_PATH forces QLinearConv's route (1 direct,
-    // 2 pixel GEMM, 3 im2col GEMM). -1 / 0 / false: not set.
+    // 2 pixel GEMM, 3 im2col GEMM, 4 depthwise kernels). -1 / 0 / false: not set.
     int force_gemm_cfg = -1;
     int force_gemv_cfg = 0;
     int i8g_rows = 0;

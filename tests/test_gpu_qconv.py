@@ -172,6 +172,20 @@ def test_depthwise_strips(sess, case):
         np.testing.assert_array_equal(got, oracle.qlinear_conv(x, zx, wt, bias, mult, zy, y_u8, **kw_))
 
 
+@pytest.mark.parametrize("case", DEPTHWISE_CASES, ids=[f"d{i}" for i in range(len(DEPTHWISE_CASES))])
+def test_depthwise_strips_forced(env_session, case):
+    """The same cases where the depthwise kernels take every form they hold, however small."""
+    n, g, h, w, mult_c, kh, kw, st, dl, pads = case
+    announce(f"qconv depthwise forced {case}")
+    rng = np.random.default_rng(sum(case[:7]) + 1)
+    qs = env_session(INGOT_QCONV_PATH=4)
+    for x_dtype, zx, y_u8, zy, with_bias in [(np.uint8, 131, True, 9, True), (np.int8, 127, False, -5, False)]:
+        x, zx, wt, bias, mult, *_ = make_case(rng, n, g, h, w, g * mult_c, kh, kw, g, x_dtype, zx, with_bias)
+        kw_ = dict(group=g, strides=st, dilations=dl, pads=pads)
+        got = run_conv(qs, x, zx, wt, bias, mult, zy, y_u8, **kw_)
+        np.testing.assert_array_equal(got, oracle.qlinear_conv(x, zx, wt, bias, mult, zy, y_u8, **kw_))
+
+
 # Pixel GEMM: channels around whole 16-byte chunks, images narrower than a word and wider than a tile, groups whose
 # channels pad, pads past the image, strides that skip columns, several images, a reduction of many k-tiles and one past
 # the chunk table (which falls back to im2col).
@@ -200,6 +214,46 @@ def test_pixel_gemm(env_session, path, case):
         kw_ = dict(group=g, strides=st, dilations=dl, pads=pads)
         got = run_conv(qs, x, zx, wt, bias, mult, zy, y_u8, **kw_)
         np.testing.assert_array_equal(got, oracle.qlinear_conv(x, zx, wt, bias, mult, zy, y_u8, **kw_))
+
+
+def conv_call(sess, n, c, h, w, m, ks, group, stride=1):
+    """A prepared u8 convolution with pad ks // 2 on random device data: the call and a function that frees it."""
+    rng = np.random.default_rng(n + c + h + m)
+    oh, ow = ((d + 2 * (ks // 2) - ks) // stride + 1 for d in (h, w))
+    wt = rng.integers(-128, 128, (m, c // group, ks, ks), dtype=np.int8)
+    pw = sess.upload_weight(wt.reshape(m, -1), trans=True, pack_dtype=L.DT_I8)
+    x = sess.to_device(rng.integers(0, 256, (n, c, h, w), dtype=np.uint8), L.DT_U8)
+    mult = sess.to_device(np.full(m, 1e-3, np.float32))
+    y = sess.empty(L.DT_U8, (n, m, oh, ow))
+
+    def call():
+        sess.qlinear_conv(x, 120, pw, wt.shape, mult, 128, y, group=group, strides=(stride, stride), pads=(ks // 2,) * 4)
+
+    return call, lambda: [t.free() for t in (pw, x, mult, y)]
+
+
+def conv_us(sess, *shape):
+    """Least time of a pass among 40, over six runs: the host's share is the same on every route."""
+    call, free = conv_call(sess, *shape)
+    best = 1e30
+    for _ in range(6):
+        sess.timer_start()
+        for _ in range(40):
+            call()
+        best = min(best, sess.timer_stop() * 1e3 / 40)
+    free()
+    return best
+
+
+@pytest.mark.parametrize("shape", [(32, 960, 7, 7, 960, 3, 960), (64, 512, 2, 2, 512, 3, 512),
+                                   (64, 512, 1, 1, 512, 1, 512), (32, 640, 7, 7, 640, 3, 640, 2),
+                                   (64, 1024, 6, 6, 1024, 3, 1024), (8, 64, 56, 56, 64, 3, 64, 3)])
+def test_small_depthwise_planes_not_slower_than_direct(env_session, shape):
+    """Depthwise planes that give a strip's wave little to do take the direct kernel (the strip kernel needed 1.6 to 7
+    times its time here)."""
+    announce(f"qconv depthwise route times {shape}")
+    auto, direct = (conv_us(env_session(INGOT_QCONV_PATH=p), *shape) for p in (0, 1))
+    assert auto < 1.3 * direct, f"{auto:.1f} us, direct {direct:.1f}"
 
 
 def test_empty_and_degenerate(sess):
