@@ -117,7 +117,10 @@ template <int KD> constexpr int pack_esz() { return KD == KIND_F32 ? 4 : (KD == 
 // Source rows are k-contiguous ([n][k]): a thread converts one 16-byte chunk
 // of a destination row, 2^txs threads side by side on a row and 256 >> txs
 // rows per workgroup, so short rows (an attention head) fill a workgroup too
-// and no thread divides.
+// and no thread divides. Few long rows are spread over gridDim.z workgroups
+// each: with one per row, the chunks of a thread follow one another at a load's
+// latency (the hi/lo planes of 64 × 11008 took 10.3 µs on MI355X, 5.8 spread; of 17 ×
+// 11008 7.9 and 4.9; bf16 of 128 × 11008 7.0 and 5.4).
 template <int KD, typename S>
 __global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p, int txs) {
     constexpr int EPC = PackOf<KD>::EPC;
@@ -127,7 +130,7 @@ __global__ __launch_bounds__(256) void pack_rows_kernel(PackArgs p, int txs) {
     char* dst = (char*)p.dst + (int64_t)blockIdx.y * p.dst_item * pack_esz<KD>();
     for (int64_t j = (int64_t)blockIdx.x * rows + ty; j < p.np; j += (int64_t)gridDim.x * rows) {
         const int64_t kin = j < p.n ? p.k : 0;
-        for (int64_t k0 = (int64_t)tx * EPC; k0 < p.kp; k0 += (int64_t)EPC << txs) {
+        for (int64_t k0 = ((int64_t)blockIdx.z << txs | tx) * EPC; k0 < p.kp; k0 += (int64_t)gridDim.z * EPC << txs) {
             Chunk<KD, S> c;
             c.load(src + j * p.ld + k0, kin - k0);
             store_chunk<KD, S>(c.v, kin - k0, p, dst + (j * p.ldk + k0) * pack_esz<KD>());
@@ -207,7 +210,11 @@ hipError_t launch_pack(const PackArgs& p, bool rows, int items, hipStream_t st) 
     if (rows) {
         int txs = 0;
         while (txs < 8 && ((int64_t)PackOf<KD>::EPC << txs) < p.kp) ++txs;
-        hipLaunchKernelGGL((pack_rows_kernel<KD, S>), dim3(grid_for(p.np, 256 >> txs), items), dim3(256), 0, st, p, txs);
+        // one step of 256 chunks a workgroup, until the chip has enough of them (eight workgroups a CU)
+        const int64_t wgs = (int64_t)grid_for(p.np, 256 >> txs) * items, steps = (p.kp / PackOf<KD>::EPC + (1 << txs) - 1) >> txs;
+        const unsigned spread = (unsigned)std::max<int64_t>(1, std::min(steps, 2048 / wgs));
+        hipLaunchKernelGGL((pack_rows_kernel<KD, S>), dim3(grid_for(p.np, 256 >> txs), items, spread), dim3(256), 0, st, p,
+                           txs);
     } else {
         const int64_t tiles_k = (p.kp + pack_tk<S>() - 1) / pack_tk<S>(), tiles = (p.np + 63) / 64 * tiles_k;
         hipLaunchKernelGGL((pack_cols_kernel<KD, S>), dim3(grid_for(tiles, 1), items), dim3(256), 0, st, p, tiles,

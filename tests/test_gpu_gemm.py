@@ -307,6 +307,40 @@ def test_weight_pack_orders(sess, n, k):
         np.testing.assert_array_equal(y.numpy(), oracle.matmul_integer(qa, qw, 131))
 
 
+@pytest.mark.parametrize("m,k", [(1, 1025), (17, 2049), (17, 11008), (70, 11003), (300, 4104), (2100, 2100)])
+def test_activation_pack_long_rows(sess, m, k):
+    """Activations whose rows are spread over several workgroups of the pack (and rows enough that they are not): the
+    bits of the same A stored [K,M], which the transposing pack takes, for every kind."""
+    announce(f"activation pack {m}x{k}")
+    rng = np.random.default_rng(m + k)
+    n = 40
+    a = rng.uniform(-1, 1, (m, k)).astype(np.float32)
+    w = rng.uniform(-1, 1, (n, k)).astype(np.float32)
+    pad = np.zeros((m, k + 3), np.float32)
+    pad[:, :k] = a
+    da, dat = sess.to_device(pad), sess.to_device(np.ascontiguousarray(a.T))
+    for pack, math in ((L.DT_F32, L.MATH_AUTO), (L.DT_BF16, L.MATH_AUTO), (L.DT_BF16, L.MATH_BF16)):
+        if pack == L.DT_BF16 and m <= 16:
+            continue  # the GEMV's rows
+        wt = sess.upload_weight(w, trans=True, pack_dtype=pack)
+        ys = []
+        for x, ta, lda in ((da, False, k + 3), (dat, True, m)):
+            y = sess.empty(L.DT_F32, (m, n))
+            sess.gemm(x, wt, y, m, trans_a=ta, lda=lda, math=math)
+            ys.append(y.numpy())
+        wt.free()
+        np.testing.assert_array_equal(ys[0], ys[1])
+        if math == L.MATH_AUTO:
+            wf = w if pack == L.DT_F32 else oracle.bf16_to_f32(oracle.f32_to_bf16(w))
+            assert_close(ys[0][:4], oracle.gemm(a[:4], wf, trans_b=True), nstar_tol(k, a, wf), f"pack {pack}")
+    qa = rng.integers(0, 256, (m, k)).astype(np.uint8)
+    qw = rng.integers(-127, 128, (k, n)).astype(np.int8)
+    wt = sess.upload_weight(qw, trans=False, pack_dtype=L.DT_I8)
+    y = sess.empty(L.DT_I32, (m, n))
+    sess.matmul_integer(sess.to_device(qa, L.DT_U8), wt, m, 131, y_i32=y)
+    np.testing.assert_array_equal(y.numpy(), oracle.matmul_integer(qa, qw, 131))
+
+
 def test_gemm_dynamic_b_decode_route(sess):
     """M <= 16, one item, bf16 B: the per-call packed B takes the GEMV route."""
     announce("gemm dynamic b gemv route")
