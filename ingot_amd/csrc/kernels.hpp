@@ -190,11 +190,11 @@ hipError_t launch_qconv_direct(const void* x, int x_u8, const QconvGeom& g, cons
                                const int32_t* bias, const float* mult, int32_t zx, float zy, int y_u8, void* y,
                                hipStream_t st);
 // Depthwise QLinearConv (g.Cg == 1); *done says whether its kernels hold this
-// form and are the faster ones (else nothing was launched and the direct kernel
-// serves it). any: every form they hold.
+// form and are faster (else nothing was launched) than the direct kernel
+// (against 0) or the GEMM too (1); against 2: every form they hold.
 hipError_t launch_qconv_depthwise(const void* x, int x_u8, const QconvGeom& g, const int8_t* w, int64_t ldw,
                                   const int32_t* bias, const float* mult, int32_t zx, float zy, int y_u8, void* y,
-                                  hipStream_t st, bool any, bool* done);
+                                  hipStream_t st, int against, bool* done);
 hipError_t launch_dequant(const void* x, int x_dtype, int64_t n, const float* scale, int64_t n_scale, int64_t inner,
                           const void* zp, int zp_dtype, int64_t n_zp, float* y, hipStream_t st);
 hipError_t launch_activation(const float* x, float* y, int64_t rows, int64_t cols, const float* bias, int act,

@@ -529,8 +529,9 @@ constexpr int DW_LDS = 64 * 1024;
 
 hipError_t launch_qconv_depthwise(const void* x, int x_u8, const QconvGeom& g, const int8_t* w, int64_t ldw,
                                   const int32_t* bias, const float* mult, int32_t zx, float zy, int y_u8, void* y,
-                                  hipStream_t st, bool any, bool* done) {
+                                  hipStream_t st, int against, bool* done) {
     *done = false;
+    const bool any = against == 2;
     // what the kernel's windows and 16-bit index arithmetic hold; anything else is the direct kernel's
     if (g.Cg != 1 || g.KW > 8 || g.dw != 1 || g.KH > 64 || g.W >= (1 << 15) || g.OW >= (1 << 15) || g.pl >= (1 << 12) ||
         g.sw > (1 << 10) || (int64_t)g.N * g.M >= (1 << 30))
@@ -597,6 +598,12 @@ hipError_t launch_qconv_depthwise(const void* x, int x_u8, const QconvGeom& g, c
                  (int64_t)p.planes * g.OH * g.OW * (13 + taps) + 284000 * taps < 6800000 ||
                  taps < 16 * (int64_t)(std::max(g.sh, g.sw) - 1)))
         return hipSuccess;
+    // Channel multipliers of 16 and more have the GEMM, too: it is ahead where the strips are too few for the chip,
+    // or small while each channel has enough outputs to fill its tiles (strip / GEMM µs, 7 × 7: 1 × 1 × 224 × 224 → 32
+    // stride 2 11.6 / 9.7, 8 images 19.9 / 31.8; 4 × 1 × 64 × 64 → 64 9.1 / 11.1, stride 2 11.5 / 8.3; 1 × 64 × 28 × 28 →
+    // 1024 10.0 / 18.3; 32 × 4 × 14 × 14 → 512 20.2 / 18.0, stride 2 19.5 / 11.6; 8 × 1 × 224 × 224 → 32 stride 4 16.6 /
+    // 13.8).
+    if (against == 1 && (items < 1024 || std::max(g.sh, g.sw) > 3 || (p.mg >= 64 && outs < 400))) return hipSuccess;
 #define INGOT_DW(SW, NWD) hipLaunchKernelGGL((qconv_dw_kernel<SW, NWD>), grid, dim3(256), lds, st, p)
     if (nwd == 1) {
         if (g.sw == 1) INGOT_DW(1, 1);

@@ -917,6 +917,43 @@ static int64_t conv_out(int64_t in, int64_t k, int64_t stride, int64_t dil, int6
     return (in + pa + pb - (dil * (k - 1) + 1)) / stride + 1;
 }
 
+// The pixel GEMM's operands: the padded channel-innermost activations of ipc
+// images at a time and the taps-outermost weight, both in the workspace.
+struct PixelGeom {
+    int64_t cgp, kt, hp, wp, img_bytes, ipc, xt_bytes, ldp, ws_bytes;
+    bool ok;  // what the chunk table, the 32-bit offsets and the layout's grid hold
+};
+
+static PixelGeom pixel_geom(const ingot_rocm_qconv_args* a, int64_t OH, int64_t OW) {
+    PixelGeom p;
+    memset(&p, 0, sizeof p);
+    const int64_t taps = a->kh * a->kw, lim = (int64_t)1 << 30;
+    p.cgp = round_up(a->c / a->group, 16);
+    p.kt = (taps * p.cgp + 127) / 128;
+    p.hp = (OH - 1) * a->stride_h + (a->kh - 1) * a->dilation_h + 1;
+    p.wp = (OW - 1) * a->stride_w + (a->kw - 1) * a->dilation_w + 1;
+    p.ldp = p.kt * 128 + 128;
+    const int64_t pitch = a->group * p.cgp;
+    if ((p.kt + 6) * 8 > CONV_CHUNKS || p.hp >= lim || p.wp >= lim || p.hp * p.wp >= lim / pitch || (a->m + 256) * p.ldp >= lim)
+        return p;
+    p.img_bytes = p.hp * p.wp * pitch;
+    const int64_t tiles = p.hp * ((p.wp + 63) / 64) * ((pitch + 63) / 64);  // of the layout launch, per image
+    if (tiles >= ((int64_t)1 << 23)) return p;
+    p.ipc = std::max<int64_t>(1, std::min({(int64_t)a->n, ((int64_t)512 << 20) / p.img_bytes, ((int64_t)1 << 22) / tiles}));
+    p.xt_bytes = round_up(p.ipc * p.img_bytes, 256);
+    p.ws_bytes = p.xt_bytes + a->m * p.ldp;
+    p.ok = true;
+    return p;
+}
+
+// Whether the workspace holds `bytes` or may be grown now (an allocation and a
+// synchronisation, which a capture refuses).
+static bool ws_at_hand(ingot_rocm_session* s, int64_t bytes) {
+    if ((size_t)bytes <= s->ws_bytes) return true;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+}
+
 int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* a, const ingot_rocm_weight* w) {
     int rc = session_enter(s);
     if (rc) return rc;
@@ -955,32 +992,39 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
     g.dh = (int)a->dilation_h, g.dw = (int)a->dilation_w, g.pt = (int)a->pad_top, g.pl = (int)a->pad_left;
     g.OH = (int)OH, g.OW = (int)OW;
     const int yu8 = a->y_dtype == INGOT_DT_U8 ? 1 : 0;
-    // Route: a GEMM needs output channels to fill MFMA tiles; depthwise and
-    // narrow groups run direct, and so do short reductions of few outputs, where
-    // one launch beats the layout and the GEMM (on MI355X, kernels alone, direct /
-    // GEMM: 4 × 128 × 28 × 28 outputs of K = 3 5.7 / 7.4 µs, of K = 19 12.4 / 8.0;
-    // 8 × 32 × 32 × 32 of K = 27 9.2 / 8.1: the line is 2^22 products).
+    // Route. Depthwise: its own kernels. Else a GEMM needs output channels to
+    // fill MFMA tiles: narrow groups run direct, and so do short reductions of
+    // few outputs, where one launch beats the layout and the GEMM (on MI355X,
+    // kernels alone, direct / pixel GEMM: 4 × 128 × 28 × 28 outputs of K = 3 5.7 /
+    // 7.4 µs, of K = 19 12.4 / 8.0; 8 × 32 × 32 × 32 of K = 27 9.2 / 8.1: the line
+    // is 2^22 products; two channels, padded to 16, pay at twice that: 4 × 16 × 64 ×
+    // 64 of K = 18 7.3 / 7.9, 4 × 32 × 64 × 64 10.4 / 8.4). A short reduction takes
+    // the GEMM only where the pixel GEMM holds it and needs no allocation inside a
+    // capture; the direct kernel needs neither.
     // INGOT_QCONV_PATH=1/2/3/4 forces direct / pixel GEMM / im2col GEMM / the
     // depthwise kernels wherever they hold the form (tests run the routes on the
     // same cases).
     const int path = s->qconv_path;
     const int64_t kgl = round_up(K, 128);
-    const bool gemm = path == 2 || path == 3 || (path == 0 && Mg >= 16 && (K >= 32 || total * K >= (1ll << 22)));
+    const PixelGeom px = pixel_geom(a, OH, OW);
+    const bool wide = path == 2 || path == 3 || (path == 0 && Mg >= 16 && K >= 32);
+    const bool gemm = wide || (path == 0 && Mg >= 16 && Cg > 1 && px.ok && total * K >= (Cg > 2 ? 1 << 22 : 1 << 23) &&
+                               ws_at_hand(s, px.ws_bytes));
+    if (wide && ((P + 256) * kgl >= lim || (w->np + 256) * w->ldk >= lim))
+        return fail(INGOT_EDECLINED, "qlinear_conv: column matrix or weight larger than 2 GiB");
+    if (Cg == 1 && (path == 0 || path == 4)) {
+        bool done = false;
+        hipError_t e = launch_qconv_depthwise(a->d_x, u8 ? 1 : 0, g, (const int8_t*)w->data, w->ldk, a->d_bias, a->d_mult,
+                                              a->zx, (float)a->zy, yu8, a->d_y, s->stream, path == 4 ? 2 : wide, &done);
+        if (e != hipSuccess) return hip_fail(e, "qconv depthwise");
+        if (done) return INGOT_OK;
+    }
     if (!gemm) {
-        if (path != 1) {
-            bool done = false;
-            hipError_t e = launch_qconv_depthwise(a->d_x, u8 ? 1 : 0, g, (const int8_t*)w->data, w->ldk, a->d_bias,
-                                                  a->d_mult, a->zx, (float)a->zy, yu8, a->d_y, s->stream, path == 4, &done);
-            if (e != hipSuccess) return hip_fail(e, "qconv depthwise");
-            if (done) return INGOT_OK;
-        }
         hipError_t e = launch_qconv_direct(a->d_x, u8 ? 1 : 0, g, (const int8_t*)w->data, w->ldk, a->d_bias,
                                            a->d_mult, a->zx, (float)a->zy, yu8, a->d_y, s->stream);
         if (e != hipSuccess) return hip_fail(e, "qconv direct");
         return INGOT_OK;
     }
-    if ((P + 256) * kgl >= lim || (w->np + 256) * w->ldk >= lim)
-        return fail(INGOT_EDECLINED, "qlinear_conv: column matrix or weight larger than 2 GiB");
     GemmArgs ga;
     memset(&ga, 0, sizeof ga);
     ga.N = (int)Mg;
@@ -1008,46 +1052,35 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
     // Pixel GEMM: the padded channel-innermost copy of x in place of the column
     // matrix, which repeats every input byte once per tap (1 × 256 × 56 × 56 →
     // 256, 3 × 3, on MI355X: im2col 24.3 + GEMM 12.6 µs; layout 4.0 + GEMM 10.2).
-    const int64_t taps = a->kh * a->kw, cgp = round_up(Cg, 16), kt_px = (taps * cgp + 127) / 128;
-    const int64_t hp = (OH - 1) * a->stride_h + (a->kh - 1) * a->dilation_h + 1;
-    const int64_t wp = (OW - 1) * a->stride_w + (a->kw - 1) * a->dilation_w + 1;
-    const int64_t px_bytes = a->group * cgp, ldp = kt_px * 128 + 128;
-    if (path != 3 && (kt_px + 6) * 8 <= CONV_CHUNKS && hp * wp < ((int64_t)1 << 30) / px_bytes &&
-        (a->m + 256) * ldp < ((int64_t)1 << 30)) {
-        const int64_t img_bytes = hp * wp * px_bytes;
-        const int64_t tiles = hp * ((wp + 63) / 64) * ((px_bytes + 63) / 64);  // of the layout launch, per image
-        const int64_t ipc = std::max<int64_t>(
-            1, std::min({(int64_t)a->n, ((int64_t)512 << 20) / img_bytes, ((int64_t)1 << 22) / tiles}));
-        if (tiles < ((int64_t)1 << 23)) {
-            const int64_t xt_bytes = round_up(ipc * img_bytes, 256);
-            void* ws;
-            rc = ws_reserve(s, (size_t)(xt_bytes + a->m * ldp), &ws);
-            if (rc) return rc;
-            int8_t* wt = (int8_t*)ws + xt_bytes;
-            ga.a = (const char*)ws;
-            ga.stride_a_bytes = cgp;
-            ga.b = (const char*)wt;
-            ga.ldb_bytes = ldp;
-            ga.stride_b_bytes = a->group > 1 ? Mg * ldp : 0;
-            ga.b_bytes = (uint32_t)((Mg - 1) * ldp + kt_px * 128);
-            ga.b_rows = (int)Mg;
-            ga.kt = (int)kt_px;
-            ga.conv = {(int)(cgp / 16), (int)taps, (int)a->kw, (int)P, (int)OW, (int)img_bytes,
-                       (int)(a->stride_h * wp * px_bytes), (int)(a->stride_w * px_bytes),
-                       (int)(a->dilation_h * wp * px_bytes), (int)(a->dilation_w * px_bytes)};
-            for (int64_t n0 = 0; n0 < a->n; n0 += ipc) {
-                const int64_t imgs = std::min(ipc, a->n - n0);
-                hipError_t e = launch_qconv_layout((const uint8_t*)a->d_x + n0 * a->c * a->h * a->w, g, (int)imgs, (int)hp,
-                                                   (int)wp, (int)cgp, (uint8_t)a->zx, u8 ? 1 : 0, ws,
-                                                   (const int8_t*)w->data, w->ldk, ldp, wt, s->stream);
-                if (e != hipSuccess) return hip_fail(e, "qconv layout");
-                ga.a_bytes = (uint32_t)(imgs * img_bytes - (a->group - 1) * cgp);
-                ga.qepi.yq = (uint8_t*)a->d_y + n0 * a->m * P;
-                e = run_rows(imgs * P);
-                if (e != hipSuccess) return hip_fail(e, "qconv gemm");
-            }
-            return INGOT_OK;
+    if (path != 3 && px.ok) {
+        void* ws;
+        rc = ws_reserve(s, (size_t)px.ws_bytes, &ws);
+        if (rc) return rc;
+        int8_t* wt = (int8_t*)ws + px.xt_bytes;
+        ga.a = (const char*)ws;
+        ga.stride_a_bytes = px.cgp;
+        ga.b = (const char*)wt;
+        ga.ldb_bytes = px.ldp;
+        ga.stride_b_bytes = a->group > 1 ? Mg * px.ldp : 0;
+        ga.b_bytes = (uint32_t)((Mg - 1) * px.ldp + px.kt * 128);
+        ga.b_rows = (int)Mg;
+        ga.kt = (int)px.kt;
+        const int64_t pitch = a->group * px.cgp;
+        ga.conv = {(int)(px.cgp / 16), (int)(a->kh * a->kw), (int)a->kw, (int)P, (int)OW, (int)px.img_bytes,
+                   (int)(a->stride_h * px.wp * pitch), (int)(a->stride_w * pitch), (int)(a->dilation_h * px.wp * pitch),
+                   (int)(a->dilation_w * pitch)};
+        for (int64_t n0 = 0; n0 < a->n; n0 += px.ipc) {
+            const int64_t imgs = std::min(px.ipc, a->n - n0);
+            hipError_t e = launch_qconv_layout((const uint8_t*)a->d_x + n0 * a->c * a->h * a->w, g, (int)imgs, (int)px.hp,
+                                               (int)px.wp, (int)px.cgp, (uint8_t)a->zx, u8 ? 1 : 0, ws,
+                                               (const int8_t*)w->data, w->ldk, px.ldp, wt, s->stream);
+            if (e != hipSuccess) return hip_fail(e, "qconv layout");
+            ga.a_bytes = (uint32_t)(imgs * px.img_bytes - (a->group - 1) * px.cgp);
+            ga.qepi.yq = (uint8_t*)a->d_y + n0 * a->m * P;
+            e = run_rows(imgs * P);
+            if (e != hipSuccess) return hip_fail(e, "qconv gemm");
         }
+        return INGOT_OK;
     }
 
     // Images per chunk: the column matrix of one chunk stays under ~512 MiB

@@ -256,6 +256,84 @@ def test_small_depthwise_planes_not_slower_than_direct(env_session, shape):
     assert auto < 1.3 * direct, f"{auto:.1f} us, direct {direct:.1f}"
 
 
+# Shapes whose route the size rules decide: channel multipliers and short reductions.
+ROUTE_SHAPES = [
+    # (n, c, h, w, m, ks, group, stride), the routes that hold it
+    ((1, 64, 28, 28, 1024, 3, 64, 1), "124"), ((4, 3, 64, 64, 96, 5, 3, 1), "124"), ((1, 8, 56, 56, 256, 7, 8, 1), "124"),
+    ((8, 3, 64, 64, 16, 1, 1, 1), "12"), ((8, 3, 128, 128, 32, 3, 1, 1), "12"),
+]
+
+
+@pytest.mark.parametrize("shape,routes", ROUTE_SHAPES, ids=[f"r{i}" for i in range(len(ROUTE_SHAPES))])
+def test_auto_route_not_slower(env_session, shape, routes):
+    """The route taken by itself against the others that hold the shape, timed in the same run."""
+    announce(f"qconv routes {shape}")
+    auto, *others = (conv_us(env_session(INGOT_QCONV_PATH=p), *shape) for p in "0" + routes)
+    assert auto < 1.2 * min(others), f"{auto:.1f} us, routes {routes}: {others}"
+
+
+@pytest.mark.parametrize("shape", [s for s, _ in ROUTE_SHAPES if s[1] * s[2] * s[3] * s[4] * s[5] ** 2 // s[6] < 4e8] +
+                         [(1, 1, 40, 41, 32, 7, 1, 4)])
+def test_routes_by_size_exact(sess, shape):
+    """The same shapes (and small ones of the same kinds) by the route taken: the oracle's bytes."""
+    announce(f"qconv route values {shape}")
+    n, c, h, w, m, ks, group, stride = shape
+    rng = np.random.default_rng(c + m)
+    x, zx, wt, bias, mult, *_ = make_case(rng, min(n, 2), c, h, w, m, ks, ks, group)
+    kw_ = dict(group=group, strides=(stride, stride), pads=(ks // 2,) * 4)
+    got = run_conv(sess, x, zx, wt, bias, mult, 17, True, **kw_)
+    np.testing.assert_array_equal(got, oracle.qlinear_conv(x, zx, wt, bias, mult, 17, True, **kw_))
+
+
+def test_short_reduction_of_a_large_image(sess):
+    """2^24 pixels with K below 32 (a column matrix would be refused): accepted, the oracle's bytes in the first and
+    last rows."""
+    announce("qconv 1 x 3 x 4096 x 4096")
+    rng = np.random.default_rng(4096)
+    x, zx, wt, bias, mult, *_ = make_case(rng, 1, 3, 4096, 4096, 16, 3, 3, 1)
+    got = run_conv(sess, x, zx, wt, bias, mult, 17, True, pads=(1, 1, 1, 1))
+    top = oracle.qlinear_conv(x[:, :, :5], zx, wt, bias, mult, 17, True, pads=(1, 1, 0, 1))
+    np.testing.assert_array_equal(got[:, :, :4], top)
+    end = oracle.qlinear_conv(x[:, :, -5:], zx, wt, bias, mult, 17, True, pads=(0, 1, 1, 1))
+    np.testing.assert_array_equal(got[:, :, -4:], end)
+
+
+def test_short_reduction_captured_on_a_fresh_session(env_session):
+    """A convolution of a short reduction captured into a graph by a session without a workspace yet: it needs none
+    there, and every replay gives the eager bytes."""
+    import ctypes
+
+    announce("qconv capture")
+    s = env_session()
+    rng = np.random.default_rng(27)
+    n, c, h, w, m = 8, 3, 64, 64, 64
+    x, zx, wt, bias, mult, *_ = make_case(rng, n, c, h, w, m, 3, 3, 1)
+    pw = s.upload_weight(wt.reshape(m, -1), trans=True, pack_dtype=L.DT_I8)
+    dx, dm, db = s.to_device(x, L.DT_U8), s.to_device(mult), s.to_device(bias)
+    y = s.empty(L.DT_U8, (n, m, h, w))
+    call = lambda: s.qlinear_conv(dx, zx, pw, wt.shape, dm, 17, y, bias=db, pads=(1, 1, 1, 1))
+    with open("/proc/self/maps") as f:
+        hip = ctypes.CDLL(next(ln.split()[-1] for ln in f if "libamdhip64" in ln))
+    st, graph, ex = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    L.check(s.lib.ingot_rocm_stream(s.h, ctypes.byref(st)))
+    s.sync()
+    assert s.workspace_bytes() == 0
+    assert hip.hipStreamBeginCapture(st, 2) == 0  # relaxed
+    call()
+    assert hip.hipStreamEndCapture(st, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+    want = oracle.qlinear_conv(x, zx, wt, bias, mult, 17, True, pads=(1, 1, 1, 1))
+    for _ in range(3):
+        s.memset(y, 0)
+        assert hip.hipGraphLaunch(ex, st) == 0
+        np.testing.assert_array_equal(y.numpy(), want)
+        s.memset(y, 0)
+        call()
+        np.testing.assert_array_equal(y.numpy(), want)
+    hip.hipGraphExecDestroy(ex)
+    hip.hipGraphDestroy(graph)
+
+
 def test_empty_and_degenerate(sess):
     announce("qconv empty")
     rng = np.random.default_rng(0)
