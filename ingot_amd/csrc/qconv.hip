@@ -1,6 +1,6 @@
 // QLinearConv on gfx950 (reference: qlinearConvOp.Run, ops/quant.go:343-420).
 //
-// Two routes, both exact in int32 and requantised with the reference's
+// Four routes, all exact in int32 and requantised with the reference's
 // expression (vek.RequantU8/I8, kernels/vek/quant_amd64.go:52-70):
 //  * pixel GEMM: one launch writes the activations channel-innermost with
 //    their padding (the zero point) and the weight with the taps outermost;
@@ -9,8 +9,9 @@
 //    channel, requantises with that channel's multiplier and stores the NCHW
 //    planes. The reference's pointwise and im2colTiled paths (:612-673).
 //  * im2col → int8 GEMM, for reductions longer than the pixel GEMM's chunk
-//    table and for groups so narrow that padding a tap's channels to 16 would
-//    lengthen them: qim2col_kernel writes, per group, the byte column matrix
+//    table and where the column matrix is estimated to cost less (few channels
+//    that pad to 16, strides that skip most pixels, more weight than columns;
+//    pixel_geom in runtime.cpp): qim2col_kernel writes, per group, the byte column matrix
 //    col[row = image·P + pixel][k = (c, kh, kw)] of the raw activations (taps
 //    outside the image hold the zero point zx, k past the group's K zero) in
 //    whole 128-byte k-tiles, the A operand of the same GEMM.

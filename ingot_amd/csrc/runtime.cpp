@@ -921,10 +921,11 @@ static int64_t conv_out(int64_t in, int64_t k, int64_t stride, int64_t dil, int6
 // images at a time and the taps-outermost weight, both in the workspace.
 struct PixelGeom {
     int64_t cgp, kt, hp, wp, img_bytes, ipc, xt_bytes, ldp, ws_bytes;
-    bool ok;  // what the chunk table, the 32-bit offsets and the layout's grid hold
+    bool ok;      // what the chunk table, the 32-bit offsets and the layout's grid hold
+    bool faster;  // than the column matrix
 };
 
-static PixelGeom pixel_geom(const ingot_rocm_qconv_args* a, int64_t OH, int64_t OW) {
+static PixelGeom pixel_geom(const ingot_rocm_qconv_args* a, int64_t OH, int64_t OW, int64_t K) {
     PixelGeom p;
     memset(&p, 0, sizeof p);
     const int64_t taps = a->kh * a->kw, lim = (int64_t)1 << 30;
@@ -943,6 +944,17 @@ static PixelGeom pixel_geom(const ingot_rocm_qconv_args* a, int64_t OH, int64_t 
     p.xt_bytes = round_up(p.ipc * p.img_bytes, 256);
     p.ws_bytes = p.xt_bytes + a->m * p.ldp;
     p.ok = true;
+    // µs on MI355X, fitted to both routes over 90 convolutions of 1–8 images. The layout: 1.2 ns a tile of 64
+    // channels × 64 columns, the weight 1 a MB (strided bytes); im2col 1.2 a MB of column matrix. Where a tap's
+    // channels pad to 16 the pixel GEMM has more k-tiles, each over all outputs, and with groups their chunks lie a
+    // pixel apart. Patches and large strides copy pixels that few taps read, and images of few pixels have more
+    // weight than columns (pixel / im2col: 8 × 3 × 224 × 224 → 768, 16 × 16 stride 16 37.9 / 16.4; 7 × 7 stride 4 → 64
+    // 21.2 / 19.4, stride 2 31.3 / 45.8; 1 × 1024 × 7 × 7 → 1024, 3 × 3 25.1 / 18.6; 1 × 256 × 14 × 14 → 256 10.1 / 11.4).
+    const double outs = (double)a->n * OH * OW * a->m, extra = (double)(p.kt - (K + 127) / 128);
+    const double layout = 3.0 + 1.2e-3 * (double)(a->n * tiles) + 1e-6 * (double)(a->m * p.kt * 128);
+    const double gemm = extra * ((a->group > 1 ? 1.5 : 0.13) + 0.25e-6 * outs);
+    const double column = 4.3 + 1.2e-6 * (double)(a->n * OH * OW * a->group) * (double)round_up(K, 128);
+    p.faster = layout + gemm < column;
     return p;
 }
 
@@ -1006,9 +1018,9 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
     // same cases).
     const int path = s->qconv_path;
     const int64_t kgl = round_up(K, 128);
-    const PixelGeom px = pixel_geom(a, OH, OW);
+    const PixelGeom px = pixel_geom(a, OH, OW, K);
     const bool wide = path == 2 || path == 3 || (path == 0 && Mg >= 16 && K >= 32);
-    const bool gemm = wide || (path == 0 && Mg >= 16 && Cg > 1 && px.ok && total * K >= (Cg > 2 ? 1 << 22 : 1 << 23) &&
+    const bool gemm = wide || (path == 0 && Mg >= 16 && Cg > 1 && px.ok && px.faster && total * K >= (Cg > 2 ? 1 << 22 : 1 << 23) &&
                                ws_at_hand(s, px.ws_bytes));
     if (wide && ((P + 256) * kgl >= lim || (w->np + 256) * w->ldk >= lim))
         return fail(INGOT_EDECLINED, "qlinear_conv: column matrix or weight larger than 2 GiB");
@@ -1052,7 +1064,7 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
     // Pixel GEMM: the padded channel-innermost copy of x in place of the column
     // matrix, which repeats every input byte once per tap (1 × 256 × 56 × 56 →
     // 256, 3 × 3, on MI355X: im2col 24.3 + GEMM 12.6 µs; layout 4.0 + GEMM 10.2).
-    if (path != 3 && px.ok) {
+    if (path != 3 && px.ok && (path == 2 || px.faster)) {
         void* ws;
         rc = ws_reserve(s, (size_t)px.ws_bytes, &ws);
         if (rc) return rc;

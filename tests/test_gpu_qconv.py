@@ -256,9 +256,12 @@ def test_small_depthwise_planes_not_slower_than_direct(env_session, shape):
     assert auto < 1.3 * direct, f"{auto:.1f} us, direct {direct:.1f}"
 
 
-# Shapes whose route the size rules decide: channel multipliers and short reductions.
+# Shapes whose route the size rules decide: patches and strides that skip pixels of few channels, a narrow first layer,
+# images of fewer pixels than the weight has rows, channel multipliers, and ordinary layers on either side.
 ROUTE_SHAPES = [
     # (n, c, h, w, m, ks, group, stride), the routes that hold it
+    ((8, 3, 224, 224, 768, 16, 1, 16), "23"), ((8, 1, 224, 224, 32, 7, 1, 4), "23"), ((8, 3, 224, 224, 64, 7, 1, 2), "23"),
+    ((1, 1024, 7, 7, 1024, 3, 1, 1), "23"), ((4, 512, 14, 14, 1024, 3, 1, 2), "23"), ((1, 256, 56, 56, 256, 3, 1, 1), "23"),
     ((1, 64, 28, 28, 1024, 3, 64, 1), "124"), ((4, 3, 64, 64, 96, 5, 3, 1), "124"), ((1, 8, 56, 56, 256, 7, 8, 1), "124"),
     ((8, 3, 64, 64, 16, 1, 1, 1), "12"), ((8, 3, 128, 128, 32, 3, 1, 1), "12"),
 ]
@@ -273,7 +276,7 @@ def test_auto_route_not_slower(env_session, shape, routes):
 
 
 @pytest.mark.parametrize("shape", [s for s, _ in ROUTE_SHAPES if s[1] * s[2] * s[3] * s[4] * s[5] ** 2 // s[6] < 4e8] +
-                         [(1, 1, 40, 41, 32, 7, 1, 4)])
+                         [(2, 3, 30, 34, 40, 16, 1, 16), (1, 1, 40, 41, 32, 7, 1, 4), (1, 520, 7, 7, 530, 3, 1, 1)])
 def test_routes_by_size_exact(sess, shape):
     """The same shapes (and small ones of the same kinds) by the route taken: the oracle's bytes."""
     announce(f"qconv route values {shape}")
