@@ -276,8 +276,10 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
 
     // CONV: the byte offset of this lane's row of each DMA instruction, and of
     // its chunk of the next k-tile to load (NW is even, so a lane has one chunk
-    // position for all its rows). Rows past M start past the buffer's end, as
-    // do chunks past the last tap (their weights are zero).
+    // position for all its rows). A row past M and a chunk past the last tap
+    // start CONV_PAST further on: either alone, and both together, lie past the
+    // buffer's end, so A reads as zero there. The sums rest on that for chunks
+    // past the last tap: nobody writes those bytes of the weight.
     static_assert(!CONV || (KD == KIND_I8 && RS == 0 && NW % 2 == 0), "CONV: int8, DMA ring");
     uint32_t pix[CONV ? IA : 1], tofs = 0;
     const uint32_t* lane_ofs = chunk_ofs + (lp ^ swz((wave & 1) * 8 + lr));
@@ -286,13 +288,13 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
         for (int q = tid; q < (p.kt + NS + 1) * 8; q += 64 * NW) {
             const int tap = q / c.cpc, kh = tap / c.kw;
             chunk_ofs[q] = tap < c.taps ? (uint32_t)(kh * c.kh_bytes + (tap - kh * c.kw) * c.kw_bytes + (q - tap * c.cpc) * 16)
-                                        : 0x80000000u;
+                                        : CONV_PAST;
         }
 #pragma unroll
         for (int j = 0; j < IA; ++j) {
             const int m = m0 + (j * NW + wave) * 8 + lr;
             const int img = m / c.p, px = m - img * c.p, oh = px / c.ow;
-            pix[j] = m < p.M ? (uint32_t)(img * c.img_bytes + oh * c.oh_bytes + (px - oh * c.ow) * c.ow_bytes) : 0x80000000u;
+            pix[j] = m < p.M ? (uint32_t)(img * c.img_bytes + oh * c.oh_bytes + (px - oh * c.ow) * c.ow_bytes) : CONV_PAST;
         }
         __syncthreads();
         tofs = lane_ofs[0];
@@ -800,7 +802,7 @@ hipError_t launch_one(const GemmArgs& a, int batch, hipStream_t st) {
     static_cast<GemmCore&>(k) = a;
     if constexpr (CONV) {
         k.conv = a.conv;
-        if ((a.kt + NS + 1) * 8 > CONV_CHUNKS) return hipErrorInvalidValue;
+        if ((a.kt + NS + 1) * 8 > CONV_CHUNKS || a.a_bytes > CONV_PAST) return hipErrorInvalidValue;
     }
     if constexpr (KD == KIND_I8)
         k.qepi = a.qepi;

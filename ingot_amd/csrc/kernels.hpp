@@ -54,6 +54,9 @@ struct ConvRows {
 // Chunk offsets a workgroup's table holds (taps · cpc rounded to k-tiles, plus
 // the k-tiles past the end that the pipeline asks for).
 constexpr int CONV_CHUNKS = 1536;
+// Added to the offset of a pixel row past the last and of a chunk past the last
+// tap: at or past every activation buffer's end, twice too (no wrap).
+constexpr uint32_t CONV_PAST = 1u << 30;
 
 // What the host fills; a launch passes the kernel only the epilogue its kind
 // reads (GemmArgsF or GemmArgsQ): the host cost of a launch grows with the

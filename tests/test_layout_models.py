@@ -150,3 +150,21 @@ def test_axis_reciprocal_quotients(d):
         for i in (q * d - 1, q * d, q * d + 1, q * d + d - 1, top):
             if 0 <= i <= top:
                 assert (((i * m) >> 32) >> (lg - 1) if lg else i) == i // d
+
+
+def test_conv_offsets_past_the_end_never_wrap():
+    """gemm_mfma.hpp CONV: with offsets inside the buffer (extent at most CONV_PAST), a row past M, a chunk past the last
+    tap and both at once give 32-bit offsets at or past the extent, where the buffer loads read zero."""
+    import os
+    import re
+
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ingot_amd", "csrc")
+    with open(os.path.join(csrc, "kernels.hpp"), encoding="utf-8") as f:
+        past = 1 << int(re.search(r"CONV_PAST = 1u << (\d+);", f.read()).group(1))
+    with open(os.path.join(csrc, "gemm_mfma.hpp"), encoding="utf-8") as f:
+        assert f.read().count("CONV_PAST;") == 2  # the row's sentinel and the chunk's
+    inside = np.array([0, 16, past // 2, past - 16], np.uint64)
+    for row, chunk in ((past, None), (None, past), (past, past)):
+        r = inside if row is None else np.array([row], np.uint64)
+        c = inside if chunk is None else np.array([chunk], np.uint64)
+        assert (((r[:, None] + c[None, :]) % (1 << 32)) >= past).all()
