@@ -245,6 +245,16 @@ def conv_us(sess, *shape):
     return best
 
 
+def assert_not_slower(env_session, shape, routes, margin):
+    """The route taken by itself takes at most margin times the best of the others (at fault only if in every attempt)."""
+    sessions = [env_session(INGOT_QCONV_PATH=p) for p in "0" + routes]
+    for _ in range(3):
+        auto, *others = (conv_us(s, *shape) for s in sessions)
+        if auto < margin * min(others):
+            return
+    raise AssertionError(f"{auto:.1f} us, routes {routes}: {others}")
+
+
 @pytest.mark.parametrize("shape", [(32, 960, 7, 7, 960, 3, 960), (64, 512, 2, 2, 512, 3, 512),
                                    (64, 512, 1, 1, 512, 1, 512), (32, 640, 7, 7, 640, 3, 640, 2),
                                    (64, 1024, 6, 6, 1024, 3, 1024), (8, 64, 56, 56, 64, 3, 64, 3)])
@@ -252,8 +262,7 @@ def test_small_depthwise_planes_not_slower_than_direct(env_session, shape):
     """Depthwise planes that give a strip's wave little to do take the direct kernel (the strip kernel needed 1.6 to 7
     times its time here)."""
     announce(f"qconv depthwise route times {shape}")
-    auto, direct = (conv_us(env_session(INGOT_QCONV_PATH=p), *shape) for p in (0, 1))
-    assert auto < 1.3 * direct, f"{auto:.1f} us, direct {direct:.1f}"
+    assert_not_slower(env_session, shape, "1", 1.3)
 
 
 # Shapes whose route the size rules decide: patches and strides that skip pixels of few channels, a narrow first layer,
@@ -271,8 +280,7 @@ ROUTE_SHAPES = [
 def test_auto_route_not_slower(env_session, shape, routes):
     """The route taken by itself against the others that hold the shape, timed in the same run."""
     announce(f"qconv routes {shape}")
-    auto, *others = (conv_us(env_session(INGOT_QCONV_PATH=p), *shape) for p in "0" + routes)
-    assert auto < 1.2 * min(others), f"{auto:.1f} us, routes {routes}: {others}"
+    assert_not_slower(env_session, shape, routes, 1.2)
 
 
 @pytest.mark.parametrize("shape", [s for s, _ in ROUTE_SHAPES if s[1] * s[2] * s[3] * s[4] * s[5] ** 2 // s[6] < 4e8] +
