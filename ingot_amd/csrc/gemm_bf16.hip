@@ -19,7 +19,7 @@ hipError_t launch_gemm_bf16(int cfg, const GemmArgs& a, int batch, hipStream_t s
         case 8: return launch_one<KIND_BF16, 64, 64, 2, 2, 4>(a, batch, st);
         // 256×192 with the weight staged through registers: every load two k-tiles ahead
         case 9: return launch_one<KIND_BF16, 256, 192, 4, 2, 2, 2>(a, batch, st);
-        case 10: return launch_one<KIND_BF16, 128, 192, 2, 4, 3>(a, batch, st);
+        case 10: return launch_one<KIND_BF16, 192, 256, 2, 4, 2>(a, batch, st);
         case 11: return launch_one<KIND_BF16, 192, 192, 4, 2, 3>(a, batch, st);
     }
     return hipErrorInvalidValue;

@@ -19,6 +19,8 @@ hipError_t launch_gemm_bf16x2(int cfg, const GemmArgs& a, int batch, hipStream_t
         case 9: return launch_one<KIND_BF16X2, 256, 192, 4, 2, 2, 2>(a, batch, st);
         case 10: return launch_one<KIND_BF16X2, 128, 192, 2, 4, 2>(a, batch, st);
         case 11: return launch_one<KIND_BF16X2, 16, 32, 1, 2, 5>(a, batch, st);
+        case 12: return launch_one<KIND_BF16X2, 192, 256, 2, 4, 2>(a, batch, st);
+        case 13: return launch_one<KIND_BF16X2, 64, 96, 2, 2, 2>(a, batch, st);
     }
     return hipErrorInvalidValue;
 }

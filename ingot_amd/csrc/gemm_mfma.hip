@@ -8,19 +8,23 @@ namespace ingot {
 namespace {
 
 // Tile configurations per kind. occupancy: workgroups per CU the LDS and
-// register footprint allow. The float kinds' costs are µs per k-tile of a round
-// of tiles that fills the chip, measured on MI355X over M = 16–4096 of the
-// decoder (2048 → 6144, 2048, 11264; 5632 → 2048), encoder (768 ↔ 3072) and
-// diffusion (3072 → 9216, 12288; 12288 → 3072) products, and pick_config adds
-// them up. A k-tile of a small tile costs its LDS traffic and its barrier, not
-// its MFMAs, so what pays is wave tiles that share fragments, eight waves (two
-// per SIMD) and three or four stages: bf16 128×128 0.35–0.43 µs with eight waves
-// and three stages against 0.57 with four waves and two, hi/lo 64×128 0.45–0.50
-// with four stages against 0.67 for two 64×64 tiles of two. Over those products
-// the tiles picked are within 0.1% (bf16) and 0.5% (hi/lo) of the best of 22 and
-// 23 measured, and 8% and 19% faster than the tables they replace (hi/lo, K =
-// 2048: 517 × 6144 42.7 → 35 µs, 1000 × 6144 83 → 48; 517 × 5632 → 2048 75 →
-// 50; bf16 2048 × 12288 → 3072 207 → 139).
+// register footprint allow. A k-tile of a small tile costs its LDS traffic and
+// its barrier, not its MFMAs, so what pays is wave tiles that share fragments,
+// eight waves (two per SIMD) and three or four stages: bf16 128×128 0.35–0.43 µs
+// with eight waves and three stages against 0.57 with four waves and two, hi/lo
+// 64×128 0.45–0.50 with four stages against 0.67 for two 64×64 tiles of two.
+// The bf16 kinds' costs (pick_config adds them up) are those that lose least
+// over 408 (bf16) and 469 (hi/lo) products, M = 17–8192, K = 64–16384, N = 64–16384
+// at random and the decoder's, encoder's and diffusion block's, every tile timed
+// on each on MI355X with the operands cached and from HBM: the picks take 0.4%
+// and 0.2% more than the best tile of each. Costs of full rounds measured on
+// forty of them, with 4 µs a round for every tile, lost up to 15% on large tiles
+// of short K and on products from HBM (hi/lo 1024 × 768 → 3072 22.9 µs, 20.9 now;
+// 4096 × 12288 → 3072 560, 512 now).
+// Tiles with two stages serve what they divide best: 192×256 (M around multiples
+// of 192: hi/lo 3000 × 4096 → 4096 181 µs against 194 with 128×128, bf16 6912 × 3256
+// → 2944 145 against 173); hi/lo 64×96, two per CU (N around multiples of 96: 1088 ×
+// 1920 → 2432 33 against 35, 1728 × 9826 → 1280 134 against 155).
 // Entry 9 is entry 1 with the weight staged through registers (gemm_kernel's
 // RS = 2): every load issued two k-tiles ahead instead of one. On MI355X, the
 // DiT MLP-down (M = 4096, N = 3072, K = 12288) right after the MLP-up GEMM
@@ -28,21 +32,21 @@ namespace {
 // 293–294, and after a 1 GiB fill 241 instead of 310; with its operands
 // already cached it is 8–12% slower (249 vs 230 µs), so the runtime takes it
 // only for products whose operands are too large to stay cached.
-const GemmConfig kBF16Cfgs[] = {{256, 256, 1, 0.f, false, -1, {1.600f}},
-                                {256, 192, 1, 0.f, false, 9, {1.294f}},
-                                {128, 128, 1, 0.f, false, -1, {0.435f}},
-                                {192, 128, 1, 0.f, false, -1, {0.633f}},
-                                {64, 128, 1, 0.f, false, -1, {0.251f}},
-                                {32, 64, 3, 0.f, false, -1, {0.141f, 0.280f, 0.381f}},
-                                {128, 256, 1, 0.f, false, -1, {0.913f}},
-                                {32, 32, 3, 0.f, false, -1, {0.124f, 0.166f, 0.264f}},
-                                {64, 64, 2, 0.f, false, -1, {0.190f, 0.351f}},
-                                {256, 192, 1, 0.f, false},
-                                {128, 192, 1, 0.f, false, -1, {0.709f}},
-                                {192, 192, 1, 0.f, false, -1, {0.911f}}};
+const GemmConfig kBF16Cfgs[] = {{256, 256, 1, -1, 0.65f, {1.380f}},
+                                {256, 192, 1, 9, 0.65f, {1.120f}},
+                                {128, 128, 1, -1, 0.65f, {0.456f}},
+                                {192, 128, 1, -1, 0.67f, {0.611f}},
+                                {64, 128, 1, -1, 0.61f, {0.260f}},
+                                {32, 64, 3, -1, 1.00f, {0.140f, 0.278f, 0.381f}},
+                                {128, 256, 1, -1, 0.83f, {0.782f}},
+                                {32, 32, 3, -1, 1.00f, {0.124f, 0.170f, 0.264f}},
+                                {64, 64, 2, -1, 0.65f, {0.194f, 0.355f}},
+                                {256, 192, 1, 9, 0.66f, {1.093f}},
+                                {192, 256, 1, -1, 0.63f, {1.115f}},
+                                {192, 192, 1, -1, 0.70f, {0.799f}}};
 // hi/lo: tiles of 128 rows hold both activation planes in a stage, which costs
-// fewer operand bytes than the taller tiles' second pass over the weight (1.28
-// against 2.56 µs for 128×192 and 256×192, half the area). 16×32 with five stages
+// fewer operand bytes than the taller tiles' second pass over the weight (1.29
+// against 2.42 µs for 128×192 and 256×192, half the area). 16×32 with five stages
 // serves up to 16 rows and long K: half the activation bytes a k-tile of 32×32,
 // and one wave's chain of fragment reads and MFMAs hidden by the fragments read
 // ahead and by up to three workgroups per CU (M = 16, weights from HBM / cached:
@@ -51,18 +55,20 @@ const GemmConfig kBF16Cfgs[] = {{256, 256, 1, 0.f, false, -1, {1.600f}},
 // round of one per CU (2048 → 11264 12.5 against 13.2). 32×32 has six stages:
 // with four the loads of a k-tile come too late (M = 64, 5632 → 4096 28.9 / 21.4
 // → 27.8 / 20.6). 16×64, 16×48, 16×16 and eight stages were level or slower.
-const GemmConfig kBF16X2Cfgs[] = {{256, 256, 1, 0.f, false, -1, {3.110f}},
-                                  {256, 192, 1, 0.f, false, 9, {2.560f}},
-                                  {128, 128, 1, 0.f, false, -1, {0.812f}},
-                                  {64, 256, 1, 0.f, false, -1, {0.897f}},
-                                  {64, 128, 1, 0.f, false, -1, {0.505f}},
-                                  {32, 64, 2, 0.f, false, -1, {0.229f, 0.423f}},
-                                  {128, 256, 1, 0.f, false, -1, {1.551f}},
-                                  {32, 32, 2, 0.f, false, -1, {0.175f, 0.320f}},
-                                  {64, 64, 1, 0.f, false, -1, {0.373f}},
-                                  {256, 192, 1, 0.f, false},
-                                  {128, 192, 1, 0.f, false, -1, {1.280f}},
-                                  {16, 32, 3, 0.f, false, -1, {0.150f, 0.280f, 0.410f}}};
+const GemmConfig kBF16X2Cfgs[] = {{256, 256, 1, -1, 0.65f, {2.993f}},
+                                  {256, 192, 1, 9, 0.63f, {2.417f}},
+                                  {128, 128, 1, -1, 0.63f, {0.916f}},
+                                  {64, 256, 1, -1, 0.66f, {0.911f}},
+                                  {64, 128, 1, -1, 0.72f, {0.468f}},
+                                  {32, 64, 2, -1, 1.00f, {0.229f, 0.435f}},
+                                  {128, 256, 1, -1, 0.63f, {1.509f}},
+                                  {32, 32, 2, -1, 1.00f, {0.175f, 0.321f}},
+                                  {64, 64, 1, -1, 0.64f, {0.320f}},
+                                  {256, 192, 1, 9, 0.65f, {2.392f}},
+                                  {128, 192, 1, -1, 0.64f, {1.287f}},
+                                  {16, 32, 3, -1, 1.00f, {0.154f, 0.293f, 0.416f}},
+                                  {192, 256, 1, -1, 0.64f, {2.402f}},
+                                  {64, 96, 2, -1, 0.68f, {0.521f, 0.742f}}};
 // f32: a k-tile is bound by its MFMAs (a tile's area per µs of cost is 7.1–9.0
 // thousand outputs, 9.0 being 147 of the 157 TFLOP/s peak), so the tiles differ
 // little but for how they divide a product over 256 CUs; 32×32 serves products
@@ -72,13 +78,13 @@ const GemmConfig kBF16X2Cfgs[] = {{256, 256, 1, 0.f, false, -1, {3.110f}},
 // 3072 38.5 against 39.7 µs with two; 260 × 2048 → 4096 50.9 against 55.7 with
 // 32×96; 2048 × 768 → 2304 56.7 against 61). Measured like the bf16 kinds'
 // costs, over M = 16–2048; the picks are within 0.5% of the best of 18 tiles.
-const GemmConfig kF32Cfgs[] = {{128, 128, 2, 0.f, false, -1, {1.816f, 3.670f}},
-                               {128, 64, 3, 0.f, false, -1, {0.936f, 1.826f, 2.750f}},
-                               {64, 64, 3, 0.f, false, -1, {0.484f, 0.924f, 1.368f}},
-                               {32, 96, 3, 0.f, false, -1, {0.432f, 0.755f, 1.229f}},
-                               {32, 32, 3, 0.f, false, -1, {0.169f, 0.294f, 0.429f}},
-                               {32, 96, 2, 0.f, false, -1, {0.387f, 0.740f}},
-                               {64, 96, 2, 0.f, false, -1, {0.723f, 1.407f}}};
+const GemmConfig kF32Cfgs[] = {{128, 128, 2, -1, 1.00f, {1.816f, 3.670f}},
+                               {128, 64, 3, -1, 1.00f, {0.936f, 1.826f, 2.750f}},
+                               {64, 64, 3, -1, 1.00f, {0.484f, 0.924f, 1.368f}},
+                               {32, 96, 3, -1, 1.00f, {0.432f, 0.755f, 1.229f}},
+                               {32, 32, 3, -1, 1.00f, {0.169f, 0.294f, 0.429f}},
+                               {32, 96, 2, -1, 1.00f, {0.387f, 0.740f}},
+                               {64, 96, 2, -1, 1.00f, {0.723f, 1.407f}}};
 // int8 64×96: two tiles per CU at M = 1024, N = 3072 (512 tiles) instead of three 64×64 ones:
 // 9.0 vs 9.6 µs on MI355X (fewer panel re-reads through L2); 128×96, 32×96, 64×128,
 // 64×192, 32-row tiles (32×32 to 32×128) and deeper rings were slower there.
@@ -91,8 +97,10 @@ const GemmConfig kF32Cfgs[] = {{128, 128, 2, 0.f, false, -1, {1.816f, 3.670f}},
 // int8 128×128 with eight waves and four stages: 2048 × 4096 → 4096 46.1 µs
 // against 53.7 with 64×96 (128×64 and 64×128 of eight waves 47.9 and 48.8); no
 // faster than 64×96 where that is two tiles per CU (1024 × 768 → 3072 8.8 / 8.3).
-const GemmConfig kI8Cfgs[] = {{256, 256, 1, 1.00f}, {128, 128, 1, 1.10f}, {128, 64, 3, 0.70f}, {64, 64, 4, 1.00f},
-                              {64, 96, 3, 1.06f}, {32, 32, 4, 0.60f, true}, {64, 64, 2, 1.20f, true}};
+const GemmConfig kI8Cfgs[] = {{256, 256, 1, -1, 1.f, {}, 1.00f}, {128, 128, 1, -1, 1.f, {}, 1.10f},
+                              {128, 64, 3, -1, 1.f, {}, 0.70f},  {64, 64, 4, -1, 1.f, {}, 1.00f},
+                              {64, 96, 3, -1, 1.f, {}, 1.06f},   {32, 32, 4, -1, 1.f, {}, 0.60f, true},
+                              {64, 64, 2, -1, 1.f, {}, 1.20f, true}};
 
 }  // namespace
 
@@ -105,6 +113,11 @@ int gemm_configs(GemmKind kind, const GemmConfig** out) {
         default: break;
     }
     return 0;
+}
+
+const GemmModel& gemm_model(GemmKind kind) {
+    static const GemmModel bf16 = {4.08f, 5.98f}, bf16x2 = {4.05f, 5.17f}, f32 = {4.00f, 0.f};
+    return kind == KIND_BF16 ? bf16 : kind == KIND_BF16X2 ? bf16x2 : f32;
 }
 
 hipError_t launch_gemm(GemmKind kind, int cfg, const GemmArgs& a, int batch, hipStream_t st) {

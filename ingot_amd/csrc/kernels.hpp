@@ -78,15 +78,22 @@ struct GemmArgsConv : GemmArgsQ {
 
 struct GemmConfig {
     int bm, bn;
-    int occupancy;   // workgroups per CU the tile allows
-    float eff;       // relative per-CU efficiency (tile-size heuristic of the kinds without costs; 0 and no cost: never picked)
-    bool one_round;  // only when every tile is resident at once (a latency-bound shape)
-    int deep = -1;   // index of the same tile with loads issued two k-tiles ahead (operands from HBM)
-    float cost[3] = {0, 0, 0};  // measured µs per k-tile with 1, 2, 3 tiles on every CU (0: not measured, eff counts)
+    int occupancy;  // workgroups per CU the tile allows
+    int deep;       // index of the same tile with loads issued two k-tiles ahead, -1: none (its own: reached only so)
+    float alone;    // k-tile cost of a tile alone on the chip relative to a full round (less traffic and power)
+    float cost[4];  // measured µs per k-tile with 1, 2, … tiles on every CU
+    float eff = 0.f;         // int8: relative per-CU efficiency instead of costs
+    bool one_round = false;  // int8: only when every tile is resident at once
+};
+// What a kind's tiles cost besides their k-tiles: µs per round of tiles (launch
+// or refill, prologue) and per 256 × 256 outputs that a CU stores.
+struct GemmModel {
+    float round, area;
 };
 
 // Tile configurations compiled for `kind`; index used by launch_gemm.
 int gemm_configs(GemmKind kind, const GemmConfig** out);
+const GemmModel& gemm_model(GemmKind kind);
 hipError_t launch_gemm(GemmKind kind, int cfg, const GemmArgs& a, int batch, hipStream_t st);
 
 struct GemvArgs {

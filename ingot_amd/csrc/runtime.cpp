@@ -75,44 +75,59 @@ constexpr int64_t kCacheResidentBytes = (int64_t)128 << 20;
 int ktile_elems(GemmKind k) { return k == KIND_F32 ? 32 : (k == KIND_I8 ? 128 : 64); }
 int kind_size(GemmKind k) { return k == KIND_F32 ? 4 : (k == KIND_I8 || k == KIND_I8G ? 1 : 2); }
 
-// Picks the tile configuration with the least estimated time. Kinds with
-// measured costs: rounds of num_cus·occupancy tiles, each a fixed 4 µs (launch
-// or refill, prologue, store) plus kt k-tiles at the cost of its most loaded
-// CU; a round that leaves CUs idle runs the bf16 kinds' tiles up to 30% faster
-// when they are large (64×64 and up: less traffic and power per CU; both numbers
-// from the measurements the costs come from). int8: full rounds weighted by
-// area and eff. Deep-ring entries marked one_round apply only when a single round
-// holds every tile. force >= 0 (INGOT_GEMM_CFG) picks that entry when it exists.
-int pick_config(GemmKind kind, int64_t M, int64_t N, int64_t kt, int64_t batch, int num_cus, int force) {
+// ceil(v / d) for the tiles' sides, by constants (the smallest calls are bound by the host).
+uint32_t tiles_along(uint32_t v, int d) {
+    switch (d) {
+        case 16: return (v + 15) / 16;
+        case 32: return (v + 31) / 32;
+        case 64: return (v + 63) / 64;
+        case 96: return (v + 95) / 96;
+        case 128: return (v + 127) / 128;
+        case 192: return (v + 191) / 192;
+        case 256: return (v + 255) / 256;
+    }
+    return (v + (uint32_t)d - 1) / (uint32_t)d;
+}
+
+// Picks the tile configuration with the least estimated time: rounds of
+// num_cus·occupancy tiles, each with the kind's time per round, its most loaded
+// CU's stores and kt k-tiles at that CU's cost (GemmModel, GemmConfig). int8: full
+// rounds weighted by area and eff, entries marked one_round only when a single
+// round holds every tile. hbm: the operands do not stay cached between uses, so a tile that has a
+// deep variant runs as that. force >= 0 (INGOT_GEMM_CFG) picks that entry when it
+// exists.
+int pick_config(GemmKind kind, int64_t M, int64_t N, int64_t kt, int64_t batch, bool hbm, int num_cus, int force) {
     const GemmConfig* c;
     const int n = gemm_configs(kind, &c);
     if (force >= 0 && force < n) return force;
+    const GemmModel& md = gemm_model(kind);
     int best = 0;
-    double best_t = 1e300;
+    float best_t = 3e38f;
     for (int i = 0; i < n; ++i) {
-        const bool timed = c[i].cost[0] > 0.f;
-        if (!timed && c[i].eff <= 0.f) continue;  // reached only as another entry's deep variant
-        // M, N < 2^31: 32-bit quotients, and none where one round holds every
-        // tile (the smallest calls are bound by the host)
-        const int64_t tiles = (int64_t)(((uint32_t)M + c[i].bm - 1) / (uint32_t)c[i].bm) *
-                              (((uint32_t)N + c[i].bn - 1) / (uint32_t)c[i].bn) * batch;
+        if (c[i].deep == i) continue;
+        const int run = hbm && c[i].deep >= 0 ? c[i].deep : i;
+        const float* cost = c[run].cost;
+        const bool timed = cost[0] > 0.f;
+        // M, N < 2^31; no division where one round holds every tile
+        const int64_t tiles = (int64_t)tiles_along((uint32_t)M, c[i].bm) * tiles_along((uint32_t)N, c[i].bn) * batch;
         const int64_t slots = (int64_t)num_cus * c[i].occupancy;
         const int64_t rounds = tiles <= slots ? 1 : (tiles + slots - 1) / slots;
         if (c[i].one_round && rounds > 1) continue;
-        double t;
+        const int64_t last = tiles - (rounds - 1) * slots;  // 1..slots tiles in the last round
+        const int per_cu = last <= num_cus ? 1 : (int)((last + num_cus - 1) / num_cus);
+        const float area = (float)(c[i].bm * c[i].bn);
+        float t;
         if (timed) {
-            const int64_t last = tiles - (rounds - 1) * slots;  // 1..slots tiles in the last round
-            const bool large = kind != KIND_F32 && c[i].bm * c[i].bn >= 64 * 64;
-            const double fill = large && last < num_cus ? 0.7 + 0.3 * (double)last / num_cus : 1.0;
-            t = 4.0 * rounds + kt * ((rounds - 1) * (double)c[i].cost[c[i].occupancy - 1] +
-                                     c[i].cost[last <= num_cus ? 0 : (last + num_cus - 1) / num_cus - 1] * fill);
+            const float full = (float)(rounds - 1);
+            const float fill = last < num_cus ? c[run].alone + (1.f - c[run].alone) * (float)last / num_cus : 1.f;
+            t = (full + 1.f) * md.round + md.area * area * (1.f / 65536) * (full * c[i].occupancy + per_cu) +
+                (float)kt * (full * cost[c[i].occupancy - 1] + cost[per_cu - 1] * fill);
         } else {
-            const int64_t per_cu = tiles <= num_cus ? 1 : std::min<int64_t>(c[i].occupancy, (tiles + num_cus - 1) / num_cus);
-            t = (double)rounds * (double)per_cu * c[i].bm * c[i].bn / c[i].eff;
+            t = (float)rounds * (rounds > 1 ? c[i].occupancy : per_cu) * area / c[i].eff;
         }
-        if (t < best_t * 0.999) {
+        if (t < best_t * 0.999f) {
             best_t = t;
-            best = i;
+            best = run;
         }
     }
     return best;
@@ -698,15 +713,14 @@ static int gemm_core(ingot_rocm_session* s, const ingot_rocm_gemm_args* a, const
     g.y = a->d_y;
     g.ldy = a->ldy;
     g.epi = make_epi(a);
-    int cfg = pick_config(kind, a->M, a->N, g.kt, batch, s->num_cus, s->force_gemm_cfg);
-    const GemmConfig* c;
-    gemm_configs(kind, &c);
     // Operands larger than half the Infinity Cache (256 MB on MI355X) do not
     // stay cached between uses: the product's own output and its neighbours'
     // evict them, so they come from HBM, where the tile whose loads are issued
     // two k-tiles ahead is faster (the configuration tables give the figures).
-    if (s->force_gemm_cfg < 0 && c[cfg].deep >= 0 && batch * a_extent + b_size > kCacheResidentBytes)
-        cfg = c[cfg].deep;
+    const int cfg = pick_config(kind, a->M, a->N, g.kt, batch, batch * a_extent + b_size > kCacheResidentBytes, s->num_cus,
+                                s->force_gemm_cfg);
+    const GemmConfig* c;
+    gemm_configs(kind, &c);
     g.tiles_m = (int)((a->M + c[cfg].bm - 1) / c[cfg].bm);
     g.tiles_n = (int)((a->N + c[cfg].bn - 1) / c[cfg].bn);
     hipError_t e = launch_gemm(kind, cfg, g, (int)batch, s->stream);
@@ -885,7 +899,7 @@ static int qgemm(ingot_rocm_session* s, int64_t M, int64_t N, int64_t K, const v
     g.qepi.yq_u8 = yq_u8;
     g.qepi.rq_mult = rq_mult;
     g.qepi.rq_zy = rq_zy;
-    const int cfg = pick_config(KIND_I8, M, N, g.kt, 1, s->num_cus, s->force_gemm_cfg);
+    const int cfg = pick_config(KIND_I8, M, N, g.kt, 1, false, s->num_cus, s->force_gemm_cfg);
     const GemmConfig* c;
     gemm_configs(KIND_I8, &c);
     g.tiles_m = (int)((M + c[cfg].bm - 1) / c[cfg].bm);
@@ -1055,7 +1069,7 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
     gemm_configs(KIND_I8, &cf);
     const auto run_rows = [&](int64_t rows) {
         ga.M = (int)rows;
-        const int cfg = pick_config(KIND_I8, rows, Mg, ga.kt, a->group, s->num_cus, s->force_gemm_cfg);
+        const int cfg = pick_config(KIND_I8, rows, Mg, ga.kt, a->group, false, s->num_cus, s->force_gemm_cfg);
         ga.tiles_m = (int)((rows + cf[cfg].bm - 1) / cf[cfg].bm);
         ga.tiles_n = (int)((Mg + cf[cfg].bn - 1) / cf[cfg].bn);
         return launch_gemm(KIND_I8, cfg, ga, (int)a->group, s->stream);

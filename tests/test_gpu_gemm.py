@@ -481,7 +481,7 @@ def test_gemv_epilogue(sess, m):
 # ragged edges in M, N and K, with a bias and an activation in the epilogue
 # (int8: the column-sum correction and fused dequantisation). Indices follow the
 # configuration tables of gemm_mfma.hip.
-GEMM_CFGS = {"f32": range(7), "bf16": range(12), "bf16x2": range(12), "i8": range(7)}
+GEMM_CFGS = {"f32": range(7), "bf16": range(12), "bf16x2": range(14), "i8": range(7)}
 
 
 @pytest.mark.parametrize("kind,cfg", [(k, c) for k, r in GEMM_CFGS.items() for c in r])
@@ -520,6 +520,56 @@ def test_gemm_forced_tile_configs(env_session, kind, cfg, m, n, k):
                        act_code=L.ACT_GELU_ERF, **({"b_dtype": bdt} if bdt is not None else {}))
     assert_close(y.numpy(), want, nstar_tol(k, a, wide), f"{kind} cfg {cfg}")
     w.free()
+
+
+# The tile picked against others that hold the product, timed in the same run: a large default-math product from HBM (the
+# register-staged tile), rows around multiples of 192, short K over large tiles, N around multiples of 96.
+PICKS = [("bf16x2", 4096, 12288, 3072, (1, 2, 9, 10)), ("bf16x2", 3000, 4096, 4096, (0, 2, 12)),
+         ("bf16x2", 1024, 768, 3072, (2, 3, 13)), ("bf16x2", 1088, 1920, 2432, (2, 3, 13)),
+         ("bf16x2", 517, 5632, 2048, (4, 8)), ("bf16", 6912, 3256, 2944, (0, 6, 10, 11)), ("bf16", 128, 3072, 768, (5, 7, 8))]
+
+
+def picked_and_forced_us(env_session, kind, m, k, n, cfgs):
+    """Least times of the product by the tile picked and by each of cfgs, taken in turn."""
+    rng = np.random.default_rng(m + n)
+    block = rng.normal(0, 1, 1 << 16).astype(np.float32)
+    if kind == "i8":
+        a, w = np.resize(block * 40, (m, k)).astype(np.int8), np.resize(block * 40, (n, k)).astype(np.int8)
+    else:
+        a, w = np.resize(block, (m, k)), np.resize(block[::-1], (n, k))
+    runs = []
+    for cfg in (-1, *cfgs):
+        s = env_session(INGOT_GEMM_CFG=cfg)
+        pw = s.upload_weight(w, trans=True, pack_dtype=L.DT_I8 if kind == "i8" else L.DT_BF16)
+        x, y = s.to_device(a), s.empty(L.DT_F32, (m, n))
+        if kind == "i8":
+            call = s.prepare_matmul_integer(x, pw, m, 3, scale=s.to_device(np.ones(1, np.float32)), y_f32=y)
+        else:
+            call = s.prepare_gemm(x, pw, y, m, math=L.MATH_AUTO if kind == "bf16x2" else L.MATH_BF16)
+        call()
+        s.sync()
+        runs.append([s, call, 1e30, (pw, x, y)])
+    reps = 10 if 2.0 * m * k * n > 1e10 else 60
+    for _ in range(6):
+        for r in runs:
+            r[0].timer_start()
+            for _ in range(reps):
+                r[1]()
+            r[2] = min(r[2], r[0].timer_stop() * 1e3 / reps)
+    for r in runs:
+        for t in r[3]:
+            t.free()
+    return runs[0][2], [r[2] for r in runs[1:]]
+
+
+@pytest.mark.parametrize("kind,m,k,n,cfgs", PICKS, ids=[f"{p[0]}-{p[1]}-{p[2]}-{p[3]}" for p in PICKS])
+def test_picked_tile_not_slower(env_session, kind, m, k, n, cfgs):
+    announce(f"picked tile {kind} {m}x{k}x{n}")
+    for _ in range(3):  # a time is at fault only if it is so in every attempt; two runs of one tile differ by up to 5%
+        picked, forced = picked_and_forced_us(env_session, kind, m, k, n, cfgs)
+        if picked < 1.09 * min(forced):
+            return
+    raise AssertionError(f"{picked:.1f} us, {dict(zip(cfgs, forced))}")
 
 
 # The hi/lo tiles that read a k-tile's fragments one k-tile ahead, against the 128 x 128 tile, which does not (the same
