@@ -32,18 +32,18 @@ namespace {
 // 293–294, and after a 1 GiB fill 241 instead of 310; with its operands
 // already cached it is 8–12% slower (249 vs 230 µs), so the runtime takes it
 // only for products whose operands are too large to stay cached.
-const GemmConfig kBF16Cfgs[] = {{256, 256, 1, -1, 0.65f, {1.380f}},
-                                {256, 192, 1, 9, 0.65f, {1.120f}},
-                                {128, 128, 1, -1, 0.65f, {0.456f}},
-                                {192, 128, 1, -1, 0.67f, {0.611f}},
-                                {64, 128, 1, -1, 0.61f, {0.260f}},
-                                {32, 64, 3, -1, 1.00f, {0.140f, 0.278f, 0.381f}},
-                                {128, 256, 1, -1, 0.83f, {0.782f}},
-                                {32, 32, 3, -1, 1.00f, {0.124f, 0.170f, 0.264f}},
-                                {64, 64, 2, -1, 0.65f, {0.194f, 0.355f}},
-                                {256, 192, 1, 9, 0.66f, {1.093f}},
-                                {192, 256, 1, -1, 0.63f, {1.115f}},
-                                {192, 192, 1, -1, 0.70f, {0.799f}}};
+const GemmConfig kBF16Cfgs[] = {{256, 256, 1, -1, 0.65f, 5.98f, {1.380f}},
+                                {256, 192, 1, 9, 0.65f, 4.49f, {1.120f}},
+                                {128, 128, 1, -1, 0.65f, 1.50f, {0.456f}},
+                                {192, 128, 1, -1, 0.67f, 2.24f, {0.611f}},
+                                {64, 128, 1, -1, 0.61f, 0.75f, {0.260f}},
+                                {32, 64, 3, -1, 1.00f, 0.19f, {0.140f, 0.278f, 0.381f}},
+                                {128, 256, 1, -1, 0.83f, 2.99f, {0.782f}},
+                                {32, 32, 3, -1, 1.00f, 0.09f, {0.124f, 0.170f, 0.264f}},
+                                {64, 64, 2, -1, 0.65f, 0.37f, {0.194f, 0.355f}},
+                                {256, 192, 1, 9, 0.66f, 4.49f, {1.093f}},
+                                {192, 256, 1, -1, 0.63f, 4.49f, {1.115f}},
+                                {192, 192, 1, -1, 0.70f, 3.36f, {0.799f}}};
 // hi/lo: tiles of 128 rows hold both activation planes in a stage, which costs
 // fewer operand bytes than the taller tiles' second pass over the weight (1.29
 // against 2.42 µs for 128×192 and 256×192, half the area). 16×32 with five stages
@@ -55,20 +55,20 @@ const GemmConfig kBF16Cfgs[] = {{256, 256, 1, -1, 0.65f, {1.380f}},
 // round of one per CU (2048 → 11264 12.5 against 13.2). 32×32 has six stages:
 // with four the loads of a k-tile come too late (M = 64, 5632 → 4096 28.9 / 21.4
 // → 27.8 / 20.6). 16×64, 16×48, 16×16 and eight stages were level or slower.
-const GemmConfig kBF16X2Cfgs[] = {{256, 256, 1, -1, 0.65f, {2.993f}},
-                                  {256, 192, 1, 9, 0.63f, {2.417f}},
-                                  {128, 128, 1, -1, 0.63f, {0.916f}},
-                                  {64, 256, 1, -1, 0.66f, {0.911f}},
-                                  {64, 128, 1, -1, 0.72f, {0.468f}},
-                                  {32, 64, 2, -1, 1.00f, {0.229f, 0.435f}},
-                                  {128, 256, 1, -1, 0.63f, {1.509f}},
-                                  {32, 32, 2, -1, 1.00f, {0.175f, 0.321f}},
-                                  {64, 64, 1, -1, 0.64f, {0.320f}},
-                                  {256, 192, 1, 9, 0.65f, {2.392f}},
-                                  {128, 192, 1, -1, 0.64f, {1.287f}},
-                                  {16, 32, 3, -1, 1.00f, {0.154f, 0.293f, 0.416f}},
-                                  {192, 256, 1, -1, 0.64f, {2.402f}},
-                                  {64, 96, 2, -1, 0.68f, {0.521f, 0.742f}}};
+const GemmConfig kBF16X2Cfgs[] = {{256, 256, 1, -1, 0.65f, 5.17f, {2.993f}},
+                                  {256, 192, 1, 9, 0.63f, 3.88f, {2.417f}},
+                                  {128, 128, 1, -1, 0.63f, 1.29f, {0.916f}},
+                                  {64, 256, 1, -1, 0.66f, 1.29f, {0.911f}},
+                                  {64, 128, 1, -1, 0.72f, 0.65f, {0.468f}},
+                                  {32, 64, 2, -1, 1.00f, 0.16f, {0.229f, 0.435f}},
+                                  {128, 256, 1, -1, 0.63f, 2.58f, {1.509f}},
+                                  {32, 32, 2, -1, 1.00f, 0.08f, {0.175f, 0.321f}},
+                                  {64, 64, 1, -1, 0.64f, 0.32f, {0.320f}},
+                                  {256, 192, 1, 9, 0.65f, 3.88f, {2.392f}},
+                                  {128, 192, 1, -1, 0.64f, 1.94f, {1.287f}},
+                                  {16, 32, 3, -1, 1.00f, 0.04f, {0.154f, 0.293f, 0.416f}},
+                                  {192, 256, 1, -1, 0.64f, 3.88f, {2.402f}},
+                                  {64, 96, 2, -1, 0.68f, 0.48f, {0.521f, 0.742f}}};
 // f32: a k-tile is bound by its MFMAs (a tile's area per µs of cost is 7.1–9.0
 // thousand outputs, 9.0 being 147 of the 157 TFLOP/s peak), so the tiles differ
 // little but for how they divide a product over 256 CUs; 32×32 serves products
@@ -78,29 +78,31 @@ const GemmConfig kBF16X2Cfgs[] = {{256, 256, 1, -1, 0.65f, {2.993f}},
 // 3072 38.5 against 39.7 µs with two; 260 × 2048 → 4096 50.9 against 55.7 with
 // 32×96; 2048 × 768 → 2304 56.7 against 61). Measured like the bf16 kinds'
 // costs, over M = 16–2048; the picks are within 0.5% of the best of 18 tiles.
-const GemmConfig kF32Cfgs[] = {{128, 128, 2, -1, 1.00f, {1.816f, 3.670f}},
-                               {128, 64, 3, -1, 1.00f, {0.936f, 1.826f, 2.750f}},
-                               {64, 64, 3, -1, 1.00f, {0.484f, 0.924f, 1.368f}},
-                               {32, 96, 3, -1, 1.00f, {0.432f, 0.755f, 1.229f}},
-                               {32, 32, 3, -1, 1.00f, {0.169f, 0.294f, 0.429f}},
-                               {32, 96, 2, -1, 1.00f, {0.387f, 0.740f}},
-                               {64, 96, 2, -1, 1.00f, {0.723f, 1.407f}}};
-// int8 64×96: two tiles per CU at M = 1024, N = 3072 (512 tiles) instead of three 64×64 ones:
-// 9.0 vs 9.6 µs on MI355X (fewer panel re-reads through L2); 128×96, 32×96, 64×128,
-// 64×192, 32-row tiles (32×32 to 32×128) and deeper rings were slower there.
-// int8 32×32 with a four-stage ring, for products whose tiles are all resident
-// at once: M = 1–128 at K = 768–2048 took 3.8–5.3 µs instead of 4.7–6.9.
-// int8 64×64 with a four-stage ring, likewise (the pixel GEMM of 256 × 56 × 56 →
-// 256, 3 × 3: 196 tiles of 18 k-tiles, 9.8–10.4 µs instead of 13.2–14.1 with two
-// stages and 11.0 with 32×32; eight stages 10.1–11.4, eight waves 10.7: with the
-// ring this deep a k-tile costs its own operand traffic, not its latency).
-// int8 128×128 with eight waves and four stages: 2048 × 4096 → 4096 46.1 µs
-// against 53.7 with 64×96 (128×64 and 64×128 of eight waves 47.9 and 48.8); no
-// faster than 64×96 where that is two tiles per CU (1024 × 768 → 3072 8.8 / 8.3).
-const GemmConfig kI8Cfgs[] = {{256, 256, 1, -1, 1.f, {}, 1.00f}, {128, 128, 1, -1, 1.f, {}, 1.10f},
-                              {128, 64, 3, -1, 1.f, {}, 0.70f},  {64, 64, 4, -1, 1.f, {}, 1.00f},
-                              {64, 96, 3, -1, 1.f, {}, 1.06f},   {32, 32, 4, -1, 1.f, {}, 0.60f, true},
-                              {64, 64, 2, -1, 1.f, {}, 1.20f, true}};
+const GemmConfig kF32Cfgs[] = {{128, 128, 2, -1, 1.00f, 0.00f, {1.816f, 3.670f}},
+                               {128, 64, 3, -1, 1.00f, 0.00f, {0.936f, 1.826f, 2.750f}},
+                               {64, 64, 3, -1, 1.00f, 0.00f, {0.484f, 0.924f, 1.368f}},
+                               {32, 96, 3, -1, 1.00f, 0.00f, {0.432f, 0.755f, 1.229f}},
+                               {32, 32, 3, -1, 1.00f, 0.00f, {0.169f, 0.294f, 0.429f}},
+                               {32, 96, 2, -1, 1.00f, 0.00f, {0.387f, 0.740f}},
+                               {64, 96, 2, -1, 1.00f, 0.00f, {0.723f, 1.407f}}};
+// int8: costs fitted like the bf16 kinds' over 425 products (M = 1–100352, N = 16–
+// 16384, K = 64–12288, f32 and byte outputs); the picks take 0.9% more than the best
+// tile of each, where one efficiency per tile taken from a single product took up
+// to 27% more (MI355X: 4096 × 4096 → 4096 84 µs with 128×128, 70 with 256×256; 8192 ×
+// 4096 → 4096 172 / 135; 4096 × 1024 → 4096 37 / 31; 2048 × 768 → 3072 16.5, 13.7 with
+// 64×96; 2048 × 4096 → 4096 42 with 128×128, 54 with 256×256). With K this short the
+// stores count as much as the k-tiles, most for 256×256, whose CUs all store at
+// once (7744 × 67 → 16320 213 µs, 126 with 64×96). 32×32 and 64×64 with four stages
+// serve products of few tiles (M = 1–128 at K = 768–2048 3.8–5.3 µs; 196 tiles of 18
+// k-tiles 9.8–10.4, 13.2–14.1 with two stages); 128×128 has eight waves and four
+// stages. 128×96, 32×96, 64×128, 64×192, 32×64 to 32×128 and deeper rings were slower.
+const GemmConfig kI8Cfgs[] = {{256, 256, 1, -1, 0.96f, 16.66f, {1.247f}},
+                              {128, 128, 1, -1, 0.90f, 2.07f, {0.629f}},
+                              {128, 64, 3, -1, 0.79f, 1.05f, {0.554f, 0.674f, 0.904f}},
+                              {64, 64, 4, -1, 0.80f, 0.44f, {0.344f, 0.381f, 0.594f, 0.682f}},
+                              {64, 96, 3, -1, 0.85f, 0.59f, {0.428f, 0.552f, 0.758f}},
+                              {32, 32, 4, -1, 1.00f, 0.16f, {0.148f, 0.194f, 0.301f, 0.301f}},
+                              {64, 64, 2, -1, 0.82f, 0.67f, {0.270f, 0.333f}}};
 
 }  // namespace
 
@@ -115,9 +117,8 @@ int gemm_configs(GemmKind kind, const GemmConfig** out) {
     return 0;
 }
 
-const GemmModel& gemm_model(GemmKind kind) {
-    static const GemmModel bf16 = {4.08f, 5.98f}, bf16x2 = {4.05f, 5.17f}, f32 = {4.00f, 0.f};
-    return kind == KIND_BF16 ? bf16 : kind == KIND_BF16X2 ? bf16x2 : f32;
+float gemm_round_us(GemmKind kind) {
+    return kind == KIND_I8 ? 2.32f : kind == KIND_BF16 ? 4.08f : kind == KIND_BF16X2 ? 4.05f : 4.f;
 }
 
 hipError_t launch_gemm(GemmKind kind, int cfg, const GemmArgs& a, int batch, hipStream_t st) {

@@ -81,19 +81,14 @@ struct GemmConfig {
     int occupancy;  // workgroups per CU the tile allows
     int deep;       // index of the same tile with loads issued two k-tiles ahead, -1: none (its own: reached only so)
     float alone;    // k-tile cost of a tile alone on the chip relative to a full round (less traffic and power)
+    float store;    // µs to store a tile of 4-byte outputs
     float cost[4];  // measured µs per k-tile with 1, 2, … tiles on every CU
-    float eff = 0.f;         // int8: relative per-CU efficiency instead of costs
-    bool one_round = false;  // int8: only when every tile is resident at once
-};
-// What a kind's tiles cost besides their k-tiles: µs per round of tiles (launch
-// or refill, prologue) and per 256 × 256 outputs that a CU stores.
-struct GemmModel {
-    float round, area;
 };
 
 // Tile configurations compiled for `kind`; index used by launch_gemm.
 int gemm_configs(GemmKind kind, const GemmConfig** out);
-const GemmModel& gemm_model(GemmKind kind);
+// µs of a round of tiles besides their k-tiles and stores (launch or refill, prologue).
+float gemm_round_us(GemmKind kind);
 hipError_t launch_gemm(GemmKind kind, int cfg, const GemmArgs& a, int batch, hipStream_t st);
 
 struct GemvArgs {

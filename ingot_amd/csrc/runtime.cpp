@@ -91,43 +91,32 @@ uint32_t tiles_along(uint32_t v, int d) {
 
 // Picks the tile configuration with the least estimated time: rounds of
 // num_cus·occupancy tiles, each with the kind's time per round, its most loaded
-// CU's stores and kt k-tiles at that CU's cost (GemmModel, GemmConfig). int8: full
-// rounds weighted by area and eff, entries marked one_round only when a single
-// round holds every tile. hbm: the operands do not stay cached between uses, so a tile that has a
-// deep variant runs as that. force >= 0 (INGOT_GEMM_CFG) picks that entry when it
-// exists.
-int pick_config(GemmKind kind, int64_t M, int64_t N, int64_t kt, int64_t batch, bool hbm, int num_cus, int force) {
+// CU's stores (out_bytes per output) and kt k-tiles at that CU's cost (GemmConfig).
+// hbm: the operands do not stay cached between uses, so a tile that has a deep
+// variant runs as that. force >= 0 (INGOT_GEMM_CFG) picks that entry when it exists.
+int pick_config(GemmKind kind, int64_t M, int64_t N, int64_t kt, int64_t batch, int out_bytes, bool hbm, int num_cus,
+                int force) {
     const GemmConfig* c;
     const int n = gemm_configs(kind, &c);
     if (force >= 0 && force < n) return force;
-    const GemmModel& md = gemm_model(kind);
+    const float round = gemm_round_us(kind), stores = 0.25f * (float)out_bytes;
     int best = 0;
     float best_t = 3e38f;
     for (int i = 0; i < n; ++i) {
         if (c[i].deep == i) continue;
-        const int run = hbm && c[i].deep >= 0 ? c[i].deep : i;
-        const float* cost = c[run].cost;
-        const bool timed = cost[0] > 0.f;
+        const GemmConfig& r = c[hbm && c[i].deep >= 0 ? c[i].deep : i];
         // M, N < 2^31; no division where one round holds every tile
-        const int64_t tiles = (int64_t)tiles_along((uint32_t)M, c[i].bm) * tiles_along((uint32_t)N, c[i].bn) * batch;
-        const int64_t slots = (int64_t)num_cus * c[i].occupancy;
-        const int64_t rounds = tiles <= slots ? 1 : (tiles + slots - 1) / slots;
-        if (c[i].one_round && rounds > 1) continue;
-        const int64_t last = tiles - (rounds - 1) * slots;  // 1..slots tiles in the last round
+        const int64_t tiles = (int64_t)tiles_along((uint32_t)M, r.bm) * tiles_along((uint32_t)N, r.bn) * batch;
+        const int64_t slots = (int64_t)num_cus * r.occupancy;
+        const int64_t full = tiles <= slots ? 0 : (tiles - 1) / slots;  // rounds before the last
+        const int64_t last = tiles - full * slots;                      // 1..slots tiles in the last
         const int per_cu = last <= num_cus ? 1 : (int)((last + num_cus - 1) / num_cus);
-        const float area = (float)(c[i].bm * c[i].bn);
-        float t;
-        if (timed) {
-            const float full = (float)(rounds - 1);
-            const float fill = last < num_cus ? c[run].alone + (1.f - c[run].alone) * (float)last / num_cus : 1.f;
-            t = (full + 1.f) * md.round + md.area * area * (1.f / 65536) * (full * c[i].occupancy + per_cu) +
-                (float)kt * (full * cost[c[i].occupancy - 1] + cost[per_cu - 1] * fill);
-        } else {
-            t = (float)rounds * (rounds > 1 ? c[i].occupancy : per_cu) * area / c[i].eff;
-        }
+        const float fill = last < num_cus ? r.alone + (1.f - r.alone) * (float)last / num_cus : 1.f;
+        const float t = (float)(full + 1) * round + stores * r.store * (float)(full * r.occupancy + per_cu) +
+                        (float)kt * ((float)full * r.cost[r.occupancy - 1] + r.cost[per_cu - 1] * fill);
         if (t < best_t * 0.999f) {
             best_t = t;
-            best = run;
+            best = (int)(&r - c);
         }
     }
     return best;
@@ -717,8 +706,8 @@ static int gemm_core(ingot_rocm_session* s, const ingot_rocm_gemm_args* a, const
     // stay cached between uses: the product's own output and its neighbours'
     // evict them, so they come from HBM, where the tile whose loads are issued
     // two k-tiles ahead is faster (the configuration tables give the figures).
-    const int cfg = pick_config(kind, a->M, a->N, g.kt, batch, batch * a_extent + b_size > kCacheResidentBytes, s->num_cus,
-                                s->force_gemm_cfg);
+    const bool hbm = batch * a_extent + b_size > kCacheResidentBytes;
+    const int cfg = pick_config(kind, a->M, a->N, g.kt, batch, g.epi.y_bf16 ? 2 : 4, hbm, s->num_cus, s->force_gemm_cfg);
     const GemmConfig* c;
     gemm_configs(kind, &c);
     g.tiles_m = (int)((a->M + c[cfg].bm - 1) / c[cfg].bm);
@@ -899,7 +888,8 @@ static int qgemm(ingot_rocm_session* s, int64_t M, int64_t N, int64_t K, const v
     g.qepi.yq_u8 = yq_u8;
     g.qepi.rq_mult = rq_mult;
     g.qepi.rq_zy = rq_zy;
-    const int cfg = pick_config(KIND_I8, M, N, g.kt, 1, false, s->num_cus, s->force_gemm_cfg);
+    const int out_bytes = (d_y_i32 ? 4 : 0) + (d_y_f32 ? 4 : 0) + (d_yq ? 1 : 0);
+    const int cfg = pick_config(KIND_I8, M, N, g.kt, 1, out_bytes, false, s->num_cus, s->force_gemm_cfg);
     const GemmConfig* c;
     gemm_configs(KIND_I8, &c);
     g.tiles_m = (int)((M + c[cfg].bm - 1) / c[cfg].bm);
@@ -1069,7 +1059,7 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
     gemm_configs(KIND_I8, &cf);
     const auto run_rows = [&](int64_t rows) {
         ga.M = (int)rows;
-        const int cfg = pick_config(KIND_I8, rows, Mg, ga.kt, a->group, false, s->num_cus, s->force_gemm_cfg);
+        const int cfg = pick_config(KIND_I8, rows, Mg, ga.kt, a->group, 1, false, s->num_cus, s->force_gemm_cfg);
         ga.tiles_m = (int)((rows + cf[cfg].bm - 1) / cf[cfg].bm);
         ga.tiles_n = (int)((Mg + cf[cfg].bn - 1) / cf[cfg].bn);
         return launch_gemm(KIND_I8, cfg, ga, (int)a->group, s->stream);

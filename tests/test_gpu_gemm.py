@@ -526,7 +526,9 @@ def test_gemm_forced_tile_configs(env_session, kind, cfg, m, n, k):
 # register-staged tile), rows around multiples of 192, short K over large tiles, N around multiples of 96.
 PICKS = [("bf16x2", 4096, 12288, 3072, (1, 2, 9, 10)), ("bf16x2", 3000, 4096, 4096, (0, 2, 12)),
          ("bf16x2", 1024, 768, 3072, (2, 3, 13)), ("bf16x2", 1088, 1920, 2432, (2, 3, 13)),
-         ("bf16x2", 517, 5632, 2048, (4, 8)), ("bf16", 6912, 3256, 2944, (0, 6, 10, 11)), ("bf16", 128, 3072, 768, (5, 7, 8))]
+         ("bf16x2", 517, 5632, 2048, (4, 8)), ("bf16", 6912, 3256, 2944, (0, 6, 10, 11)), ("bf16", 128, 3072, 768, (5, 7, 8)),
+         ("i8", 4096, 4096, 4096, (0, 1)), ("i8", 4096, 4096, 8192, (0, 1)), ("i8", 4096, 1024, 4096, (0, 1, 2)),
+         ("i8", 2048, 768, 3072, (1, 2, 4)), ("i8", 2048, 4096, 4096, (0, 1, 4)), ("i8", 1024, 768, 3072, (3, 4))]
 
 
 def picked_and_forced_us(env_session, kind, m, k, n, cfgs):
