@@ -21,6 +21,7 @@ hipError_t launch_gemm_bf16(int cfg, const GemmArgs& a, int batch, hipStream_t s
         case 9: return launch_one<KIND_BF16, 256, 192, 4, 2, 2, 2>(a, batch, st);
         case 10: return launch_one<KIND_BF16, 192, 256, 2, 4, 2>(a, batch, st);
         case 11: return launch_one<KIND_BF16, 192, 192, 4, 2, 3>(a, batch, st);
+        case 12: return launch_one<KIND_BF16, 128, 192, 2, 4, 3>(a, batch, st);
     }
     return hipErrorInvalidValue;
 }

@@ -14,7 +14,7 @@ namespace {
 // with eight waves and three stages against 0.57 with four waves and two, hi/lo
 // 64×128 0.45–0.50 with four stages against 0.67 for two 64×64 tiles of two.
 // The bf16 kinds' costs (pick_config adds them up) are those that lose least
-// over 408 (bf16) and 469 (hi/lo) products, M = 17–8192, K = 64–16384, N = 64–16384
+// over 500 (bf16) and 469 (hi/lo) products, M = 17–8192, K = 64–16384, N = 64–16384
 // at random and the decoder's, encoder's and diffusion block's, every tile timed
 // on each on MI355X with the operands cached and from HBM: the picks take 0.4%
 // and 0.2% more than the best tile of each. Costs of full rounds measured on
@@ -24,7 +24,9 @@ namespace {
 // Tiles with two stages serve what they divide best: 192×256 (M around multiples
 // of 192: hi/lo 3000 × 4096 → 4096 181 µs against 194 with 128×128, bf16 6912 × 3256
 // → 2944 145 against 173); hi/lo 64×96, two per CU (N around multiples of 96: 1088 ×
-// 1920 → 2432 33 against 35, 1728 × 9826 → 1280 134 against 155).
+// 1920 → 2432 33 against 35, 1728 × 9826 → 1280 134 against 155). bf16 128×192 with
+// three stages has the products of one round that 192×128 and 128×128 divide worse
+// (2048 × 768 → 3072, bf16 out, 18.6 µs; 24.4 with 192×192).
 // Entry 9 is entry 1 with the weight staged through registers (gemm_kernel's
 // RS = 2): every load issued two k-tiles ahead instead of one. On MI355X, the
 // DiT MLP-down (M = 4096, N = 3072, K = 12288) right after the MLP-up GEMM
@@ -32,18 +34,19 @@ namespace {
 // 293–294, and after a 1 GiB fill 241 instead of 310; with its operands
 // already cached it is 8–12% slower (249 vs 230 µs), so the runtime takes it
 // only for products whose operands are too large to stay cached.
-const GemmConfig kBF16Cfgs[] = {{256, 256, 1, -1, 0.65f, 5.98f, {1.380f}},
-                                {256, 192, 1, 9, 0.65f, 4.49f, {1.120f}},
-                                {128, 128, 1, -1, 0.65f, 1.50f, {0.456f}},
-                                {192, 128, 1, -1, 0.67f, 2.24f, {0.611f}},
-                                {64, 128, 1, -1, 0.61f, 0.75f, {0.260f}},
-                                {32, 64, 3, -1, 1.00f, 0.19f, {0.140f, 0.278f, 0.381f}},
-                                {128, 256, 1, -1, 0.83f, 2.99f, {0.782f}},
-                                {32, 32, 3, -1, 1.00f, 0.09f, {0.124f, 0.170f, 0.264f}},
-                                {64, 64, 2, -1, 0.65f, 0.37f, {0.194f, 0.355f}},
-                                {256, 192, 1, 9, 0.66f, 4.49f, {1.093f}},
-                                {192, 256, 1, -1, 0.63f, 4.49f, {1.115f}},
-                                {192, 192, 1, -1, 0.70f, 3.36f, {0.799f}}};
+const GemmConfig kBF16Cfgs[] = {{256, 256, 1, -1, 0.61f, 5.96f, {1.341f}},
+                                {256, 192, 1, 9, 0.66f, 4.47f, {1.104f}},
+                                {128, 128, 1, -1, 0.67f, 1.49f, {0.457f}},
+                                {192, 128, 1, -1, 0.64f, 2.23f, {0.603f}},
+                                {64, 128, 1, -1, 0.60f, 0.74f, {0.264f}},
+                                {32, 64, 3, -1, 1.00f, 0.19f, {0.143f, 0.284f, 0.397f}},
+                                {128, 256, 1, -1, 0.89f, 2.98f, {0.775f}},
+                                {32, 32, 3, -1, 1.00f, 0.09f, {0.127f, 0.169f, 0.272f}},
+                                {64, 64, 2, -1, 0.73f, 0.37f, {0.195f, 0.381f}},
+                                {256, 192, 1, 9, 0.66f, 4.47f, {1.094f}},
+                                {192, 256, 1, -1, 0.64f, 4.47f, {1.112f}},
+                                {192, 192, 1, -1, 0.71f, 3.35f, {0.798f}},
+                                {128, 192, 1, -1, 0.66f, 2.23f, {0.655f}}};
 // hi/lo: tiles of 128 rows hold both activation planes in a stage, which costs
 // fewer operand bytes than the taller tiles' second pass over the weight (1.29
 // against 2.42 µs for 128×192 and 256×192, half the area). 16×32 with five stages
@@ -118,7 +121,7 @@ int gemm_configs(GemmKind kind, const GemmConfig** out) {
 }
 
 float gemm_round_us(GemmKind kind) {
-    return kind == KIND_I8 ? 2.32f : kind == KIND_BF16 ? 4.08f : kind == KIND_BF16X2 ? 4.05f : 4.f;
+    return kind == KIND_I8 ? 2.32f : kind == KIND_BF16 ? 4.06f : kind == KIND_BF16X2 ? 4.05f : 4.f;
 }
 
 hipError_t launch_gemm(GemmKind kind, int cfg, const GemmArgs& a, int batch, hipStream_t st) {

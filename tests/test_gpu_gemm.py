@@ -481,7 +481,7 @@ def test_gemv_epilogue(sess, m):
 # ragged edges in M, N and K, with a bias and an activation in the epilogue
 # (int8: the column-sum correction and fused dequantisation). Indices follow the
 # configuration tables of gemm_mfma.hip.
-GEMM_CFGS = {"f32": range(7), "bf16": range(12), "bf16x2": range(14), "i8": range(7)}
+GEMM_CFGS = {"f32": range(7), "bf16": range(13), "bf16x2": range(14), "i8": range(7)}
 
 
 @pytest.mark.parametrize("kind,cfg", [(k, c) for k, r in GEMM_CFGS.items() for c in r])
@@ -527,6 +527,7 @@ def test_gemm_forced_tile_configs(env_session, kind, cfg, m, n, k):
 PICKS = [("bf16x2", 4096, 12288, 3072, (1, 2, 9, 10)), ("bf16x2", 3000, 4096, 4096, (0, 2, 12)),
          ("bf16x2", 1024, 768, 3072, (2, 3, 13)), ("bf16x2", 1088, 1920, 2432, (2, 3, 13)),
          ("bf16x2", 517, 5632, 2048, (4, 8)), ("bf16", 6912, 3256, 2944, (0, 6, 10, 11)), ("bf16", 128, 3072, 768, (5, 7, 8)),
+         ("bf16", 2048, 768, 3072, (2, 3, 11, 12)), ("bf16", 512, 6464, 13056, (2, 6, 11)),
          ("i8", 4096, 4096, 4096, (0, 1)), ("i8", 4096, 4096, 8192, (0, 1)), ("i8", 4096, 1024, 4096, (0, 1, 2)),
          ("i8", 2048, 768, 3072, (1, 2, 4)), ("i8", 2048, 4096, 4096, (0, 1, 4)), ("i8", 1024, 768, 3072, (3, 4))]
 
