@@ -1022,10 +1022,12 @@ int ingot_rocm_qlinear_conv(ingot_rocm_session* s, const ingot_rocm_qconv_args* 
     // same cases).
     const int path = s->qconv_path;
     const int64_t kgl = round_up(K, 128);
-    const PixelGeom px = pixel_geom(a, OH, OW, K);
+    PixelGeom px;
+    px.ok = false;
+    if (path == 2 || (path == 0 && Mg >= 16)) px = pixel_geom(a, OH, OW, K);
     const bool wide = path == 2 || path == 3 || (path == 0 && Mg >= 16 && K >= 32);
-    const bool gemm = wide || (path == 0 && Mg >= 16 && Cg > 1 && px.ok && px.faster && total * K >= (Cg > 2 ? 1 << 22 : 1 << 23) &&
-                               ws_at_hand(s, px.ws_bytes));
+    const bool gemm = wide || (path == 0 && Mg >= 16 && Cg > 1 && total * K >= (Cg > 2 ? 1 << 22 : 1 << 23) && px.ok &&
+                               px.faster && ws_at_hand(s, px.ws_bytes));
     if (wide && ((P + 256) * kgl >= lim || (w->np + 256) * w->ldk >= lim))
         return fail(INGOT_EDECLINED, "qlinear_conv: column matrix or weight larger than 2 GiB");
     if (Cg == 1 && (path == 0 || path == 4)) {
