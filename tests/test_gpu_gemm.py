@@ -17,6 +17,7 @@ import oracle
 from helpers import announce, assert_close, bf16_weights, nstar_tol
 from ingot_amd import IngotError
 from ingot_amd import _lib as L
+from ingot_amd.host import DeviceTensor
 
 pytestmark = pytest.mark.gpu
 
@@ -273,6 +274,53 @@ def test_gemm_dynamic_b_in_place(sess, b_dt, m, n, k, pad):
     np.testing.assert_array_equal(got, product(k, n, np.ascontiguousarray(bits.transpose(0, 2, 1)), False, 0))
     for i in range(bsz):
         assert_close(got[i], oracle.gemm(a[i], bt[i], trans_b=True), nstar_tol(k, a, bt), f"in place item {i}")
+
+
+@pytest.mark.parametrize("b_dt", ["f32", "bf16"])
+@pytest.mark.parametrize("start", [0, 4096, 70 * 128 * 2 - 1024])
+def test_gemm_dynamic_b_output_over_b(sess, b_dt, start):
+    """Y written over a B whose form could be read in place (`start` bytes into it, so that the first, the inner or the
+    last bytes of B are overwritten): the bits of the product with a Y of its own."""
+    announce(f"gemm dynamic b with Y over B {b_dt} {start}")
+    rng = np.random.default_rng(start + len(b_dt))
+    m, n, k = 33, 70, 128
+    a = rng.uniform(-1, 1, (m, k)).astype(np.float32)
+    bt = rng.uniform(-1, 1, (n, k)).astype(np.float32)
+    bits = oracle.f32_to_bf16(bt) if b_dt == "bf16" else bt
+    dt = L.DT_BF16 if b_dt == "bf16" else L.DT_F32
+    da, db, y = sess.to_device(a), sess.to_device(bits, dt), sess.empty(L.DT_F32, (m, n))
+    sess.gemm_dynamic_b(da, db, y, m, n, k, True, k, 0)
+    want = y.numpy()
+    room = sess.to_device(np.zeros(1 << 17, np.uint8), L.DT_U8)
+    over_b = DeviceTensor(sess, dt, (n, k), room.ptr, False)
+    over_y = DeviceTensor(sess, L.DT_F32, (m, n), room.ptr + start, False)
+    L.check(sess.lib.ingot_rocm_memcpy_h2d(sess.h, over_b.ptr, np.ascontiguousarray(bits).ctypes.data, bits.nbytes))
+    assert start < bits.nbytes
+    sess.gemm_dynamic_b(da, over_b, over_y, m, n, k, True, k, 0)
+    np.testing.assert_array_equal(over_y.numpy(), want)
+
+
+# Up to 16 rows of default math by wide bf16 weights, the work of the 16 x 32 tile: K within one k-tile, the five of
+# its ring and many more (odd and even, ragged), N off the tile; the 128 x 128 tile sums in the same order.
+@pytest.mark.parametrize("m", [5, 11, 16])
+def test_gemm_few_rows_wide_equal_bits(env_session, m):
+    announce(f"gemm few rows wide m={m}")
+    rng = np.random.default_rng(m)
+    auto, ref, tile = env_session(), env_session(INGOT_GEMM_CFG=2), env_session(INGOT_GEMM_CFG=11)
+    for n, k in [(4096, 64), (4100, 320), (4127, 321), (6144, 2048), (4097, 5632), (4096, 1000)]:
+        a, bt = rng.normal(0, 1, (m, k)).astype(np.float32), bf16_weights(rng, (n, k))
+        out = []
+        for s in (auto, ref, tile):
+            w = s.upload_weight(bt, trans=True, pack_dtype=L.DT_BF16, src_dtype=L.DT_BF16)
+            y = s.empty(L.DT_F32, (m, n))
+            s.gemm(s.to_device(a), w, y, m)
+            out.append(y.numpy())
+            w.free()
+        np.testing.assert_array_equal(out[0], out[1])
+        np.testing.assert_array_equal(out[2], out[1])
+        cols = np.r_[0:40, n - 40:n]
+        want = oracle.gemm(a, bt[cols], trans_b=True, b_dtype=oracle.BF16)
+        assert_close(out[0][:, cols], want, nstar_tol(k, a, oracle.bf16_to_f32(bt)), f"few rows {m}x{k}x{n}")
 
 
 @pytest.mark.parametrize("n,k", [(1, 1), (63, 65), (64, 64), (65, 63), (130, 257), (257, 128)])

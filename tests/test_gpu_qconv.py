@@ -3,9 +3,9 @@
 Bar: bit-exact against the oracle's restatement of the reference
 (qlinearConvOp.Run, ops/quant.go:343-706), on the geometries of the
 reference's TestQLinearConv (ops/quant_optest_test.go:133-192) and on larger
-shapes that take the im2col → int8 MFMA GEMM route. Both device routes
-(direct, GEMM) run every case: INGOT_QCONV_PATH=1 forces the direct kernel,
-2 the GEMM.
+shapes that take an int8 MFMA GEMM. Every device route runs every case:
+INGOT_QCONV_PATH=1 forces the direct kernel, 2 the pixel GEMM, 3 im2col and
+the GEMM over its column matrix; 4 the depthwise kernels wherever they hold.
 """
 
 import numpy as np
@@ -22,7 +22,7 @@ pytestmark = pytest.mark.gpu
 DT = {np.dtype(np.uint8): L.DT_U8, np.dtype(np.int8): L.DT_I8}
 
 
-ROUTES = {"auto": "0", "direct": "1", "gemm": "2"}
+ROUTES = {"auto": "0", "direct": "1", "pixel": "2", "im2col": "3"}
 
 
 @pytest.fixture(params=list(ROUTES))
@@ -214,6 +214,42 @@ def test_pixel_gemm(env_session, path, case):
         kw_ = dict(group=g, strides=st, dilations=dl, pads=pads)
         got = run_conv(qs, x, zx, wt, bias, mult, zy, y_u8, **kw_)
         np.testing.assert_array_equal(got, oracle.qlinear_conv(x, zx, wt, bias, mult, zy, y_u8, **kw_))
+
+
+# Every instance of the pixel GEMM (they differ in waves, ring depth and where the chunk table lies): pixels and channels
+# off every tile's grid, groups, several images, one k-tile and more than a ring holds.
+@pytest.mark.parametrize("cfg", range(7))
+@pytest.mark.parametrize("case", [PIXEL_CASES[i] for i in (0, 3, 4)] +
+                         [(3, 40, 11, 29, 270, 3, 3, 2, (1, 1), (1, 1), (1, 1, 1, 1)),
+                          (2, 272, 5, 9, 130, 3, 3, 1, (2, 1), (1, 1), (1, 1, 1, 1))], ids=[f"t{i}" for i in range(5)])
+def test_pixel_gemm_forced_tiles(env_session, cfg, case):
+    n, c, h, w, m, kh, kw, g, st, dl, pads = case
+    m = -(-m // g) * g
+    announce(f"qconv pixel gemm tile {cfg} {case}")
+    rng = np.random.default_rng(sum(case[:7]) + 2)
+    qs = env_session(INGOT_QCONV_PATH=2, INGOT_GEMM_CFG=cfg)
+    x, zx, wt, bias, mult, *_ = make_case(rng, n, c, h, w, m, kh, kw, g, np.uint8, 131, True)
+    kw_ = dict(group=g, strides=st, dilations=dl, pads=pads)
+    got = run_conv(qs, x, zx, wt, bias, mult, 9, True, **kw_)
+    np.testing.assert_array_equal(got, oracle.qlinear_conv(x, zx, wt, bias, mult, 9, True, **kw_))
+
+
+@pytest.mark.parametrize("path", [2, 3])
+def test_images_in_two_chunks(env_session, path):
+    """Images whose copies exceed the chunk's 512 MiB (three of 12.6 million pixels of 16 bytes; the column matrix of
+    path 3 likewise) run in chunks that share one workspace: the oracle's bytes at both ends of every image."""
+    announce(f"qconv 3 x 1 x 4096 x 3072 in chunks, path={path}")
+    rng = np.random.default_rng(3072)
+    x, zx, wt, bias, mult, *_ = make_case(rng, 3, 1, 4096, 3072, 16, 3, 3, 1)
+    qs = env_session(INGOT_QCONV_PATH=path)
+    kw_ = dict(strides=(2, 2))
+    got = run_conv(qs, x, zx, wt, bias, mult, 17, True, pads=(1, 1, 1, 1), **kw_)
+    assert 2 * 16 * 4096 * 3072 < 512 << 20 < 3 * 16 * 4096 * 3072 and got.shape == (3, 16, 2048, 1536)
+    for i in range(3):
+        top = oracle.qlinear_conv(x[i:i + 1, :, :6], zx, wt, bias, mult, 17, True, pads=(1, 1, 0, 1), **kw_)
+        np.testing.assert_array_equal(got[i:i + 1, :, :3], top)
+        end = oracle.qlinear_conv(x[i:i + 1, :, -7:], zx, wt, bias, mult, 17, True, pads=(0, 1, 0, 1), **kw_)
+        np.testing.assert_array_equal(got[i:i + 1, :, -3:], end)
 
 
 def conv_call(sess, n, c, h, w, m, ks, group, stride=1):
