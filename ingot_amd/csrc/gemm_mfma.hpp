@@ -449,7 +449,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, 1) void gemm_kernel(typename Kernel
     // register sets; the sums keep their order). On MI355X, cached operands:
     // 16×32 tile at M = 16, 5632 → 4096 19.1 → 16.9 µs; 64×128 at M = 17, 2048 →
     // 6144 19.2 → 16.7; 64×128 at M = 64, 5632 → 4096 44.4 → 38.6. Wave tiles of
-    // more blocks cover the latency with their MFMAs and would need the registers.
+    // eight blocks (128×128, 64×256: 106 VGPRs, a second set would fit) have twice the
+    // MFMAs to cover the latency and were not measured with it.
     constexpr bool AHEAD = KD == KIND_BF16X2 && AP == 2 && TM * TN <= 4;
     FragA fa0, fa1;
     FragB fb0, fb1;

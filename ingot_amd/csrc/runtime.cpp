@@ -629,9 +629,10 @@ int ingot_rocm_gemv_bf16(ingot_rocm_session* s, const ingot_rocm_gemm_args* a) {
 }
 
 // Decode rows take the GEMV: all of M <= 4, and M = 5..16 for N < 4096. At
-// M = 5..16 the wider products run faster as a GEMM of four-stage 32×32
-// tiles (on MI355X at K = 2048, M = 8 and 16: N = 6144 10.7 vs 12.7 µs, N =
-// 11264 13.1 vs 16.2 µs; N = 2048 the GEMV stays ahead, 8.7 vs 10.4 µs).
+// M = 5..16 the wider products run faster as a GEMM of 16×32 tiles, whose pre-pass and
+// k-chain cost the same however many columns there are (MI355X, default math, M = 8,
+// operands cached, GEMV / GEMM µs: K = 2048, N = 1024 7.0 / 9.3, 2048 7.3 / 9.4, 3072
+// 10.2 / 9.5, 6144 - / 9.9; K = 4096, N = 2048 13.2 / 13.2, 3072 17.5 / 13.4).
 static bool gemv_route(const ingot_rocm_session* s, const ingot_rocm_gemm_args* a, GemmKind kind) {
     return kind == KIND_BF16 && a->M <= 16 && (a->M <= 4 || a->N < 4096) && !a->trans_a &&
            a->a_dtype == INGOT_DT_F32 && a->batch <= 1 && !s->no_gemv;
