@@ -629,7 +629,7 @@ int ingot_rocm_gemv_bf16(ingot_rocm_session* s, const ingot_rocm_gemm_args* a) {
 }
 
 // Decode rows take the GEMV: all of M <= 4, and M = 5..16 for N < 4096. At
-// M = 5..16 the wider products run faster as a GEMM of 16×32 tiles, whose pre-pass and
+// M = 5..16 the wider products run faster as a GEMM of 16×32 or 32×64 tiles, whose pre-pass and
 // k-chain cost the same however many columns there are (MI355X, default math, M = 8,
 // operands cached, GEMV / GEMM µs: K = 2048, N = 1024 7.0 / 9.3, 2048 7.3 / 9.4, 3072
 // 10.2 / 9.5, 6144 - / 9.9; K = 4096, N = 2048 13.2 / 13.2, 3072 17.5 / 13.4).
