@@ -595,9 +595,11 @@ hipError_t launch_qconv_depthwise(const void* x, int x_u8, const QconvGeom& g, c
     // 14.0; 2 × 2 stride 2, 56 × 56 10.7 / 7.0, 4 × 4 10.8 / 11.4; 512 of 112 × 112
     // stride 3, 3 × 3 11.9 / 10.3, 7 × 7 16.5 / 31.0).
     const int64_t taps = (int64_t)g.KH * g.KW, outs = (int64_t)p.th * g.OW;
-    // Strips so few that one round holds them run at their latency, which 25 taps of the direct kernel exceed (672 planes
-    // of 7 × 7, 5 × 5 5.4 / 6.0).
-    const bool few = taps >= 24 && outs >= 25 && items <= 4096;
+    // Few strips run at their latency, 5.4 µs + 0.8 ns each, which 3 µs + 0.12 a tap of the direct kernel exceed unless most
+    // taps lie outside the image: up to 150·taps − 3000 strips, and 4096 of 25 outputs and more (672 planes of 7 × 7, 5 × 5
+    // 5.4 / 6.0; 7 × 7 stride 2 on 7 × 7 6.6 / 9.2, on 4 × 4 6.6 / 7.9; 3840 of 4 × 4, 7 × 7 8.1 / 9.3, 5 × 5 7.6 / 5.9; 672
+    // of 3 × 3, 7 × 7 7.6 / 6.9).
+    const bool few = taps >= 24 && std::min(g.H, g.W) >= 4 && (items <= 150 * taps - 3000 || (outs >= 25 && items <= 4096));
     if (!any && ((outs * (13 + taps) < 2000 && !few) ||
                  (int64_t)p.planes * g.OH * g.OW * (13 + taps) + 284000 * taps < 6800000 ||
                  taps < 16 * (int64_t)(std::max(g.sh, g.sw) - 1)))

@@ -302,12 +302,14 @@ def test_small_depthwise_planes_not_slower_than_direct(env_session, shape):
 
 
 # Shapes whose route the size rules decide: patches and strides that skip pixels of few channels, a narrow first layer,
-# images of fewer pixels than the weight has rows, channel multipliers, and ordinary layers on either side.
+# images of fewer pixels than the weight has rows, channel multipliers, few small depthwise planes, and ordinary layers on
+# either side.
 ROUTE_SHAPES = [
     # (n, c, h, w, m, ks, group, stride), the routes that hold it
     ((8, 3, 224, 224, 768, 16, 1, 16), "23"), ((8, 1, 224, 224, 32, 7, 1, 4), "23"), ((8, 3, 224, 224, 64, 7, 1, 2), "23"),
     ((1, 1024, 7, 7, 1024, 3, 1, 1), "23"), ((4, 512, 14, 14, 1024, 3, 1, 2), "23"), ((1, 256, 56, 56, 256, 3, 1, 1), "23"),
     ((1, 64, 28, 28, 1024, 3, 64, 1), "124"), ((4, 3, 64, 64, 96, 5, 3, 1), "124"), ((1, 8, 56, 56, 256, 7, 8, 1), "124"),
+    ((1, 672, 7, 7, 672, 7, 672, 2), "14"), ((2, 1152, 5, 5, 1152, 7, 1152, 2), "14"), ((8, 480, 4, 4, 480, 5, 480, 1), "14"),
     ((8, 3, 64, 64, 16, 1, 1, 1), "12"), ((8, 3, 128, 128, 32, 3, 1, 1), "12"),
 ]
 
